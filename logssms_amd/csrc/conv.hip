@@ -144,6 +144,7 @@ struct FrontParams {
   float* b_out;
   int64_t g_ld;  // 0: g_out / b_out [T, HV]; else head-major [HV, g_ld]
   int qk_f16;  // q_out / k_out as f16 MFMA operands (the bf16-rounded values, converted)
+  int tile;    // conv_vec_kernel: tokens per block
 };
 
 // grid: (token tiles, C / 256).  A 256-channel slab holds whole q/k heads
@@ -218,12 +219,26 @@ __global__ __launch_bounds__(kThreads) void frontend_kernel(FrontParams fp) {
 
 // ---------------------------------------------- vectorised path (8 channels / thread)
 // Used when the input rows are unit-stride, 16-byte aligned and C % 8 == 0.
-// Each thread owns 8 consecutive channels for a tile of kVTok tokens: one
-// 16-byte load and one 16-byte store per token, the W-1 previous inputs in
-// registers, and the per-head q/k sum of squares reduced across the DK/8
-// lanes of the head with cross-lane shuffles (no LDS).
-constexpr int kVTok = 32;
-
+// Each thread owns 8 consecutive channels for a tile of tokens: one 16-byte
+// load and one 16-byte store per token, the W-1 previous inputs in registers,
+// and the per-head q/k sum of squares reduced across the DK/8 lanes of the
+// head with cross-lane shuffles (no LDS).
+//
+// Tokens per block.  A block walks its tile serially, about 0.6 us a token
+// when alone on its CU, so a 32-token tile took 23-29 us at any T below 4096;
+// a shorter tile re-reads the W-1 rows before it (from L2).  The largest tile
+// that still gives the chip kConvBlocks blocks (2.75 per CU) is within 8 % of
+// the fastest one measured at each T (q/k pass, 2 slabs, us at tile 32 / 16 /
+// 8 / 4 / 2): T 300: 23.8 / 13.5 / 9.0 / 6.7 / 5.8; 2048: 28.9 / 15.9 / 13.1 /
+// 13.2 / 15.9; 8192: 36.8 / 30.3 / 30.8 / 35.8 / 45.0; 16384: 63.4 / 64.4 /
+// 65.7 / 70.5 / 87.8.
+constexpr int kVTok = 32, kVTokMin = 2;
+constexpr int64_t kConvBlocks = 704;
+inline int conv_tile(int64_t tokens, int64_t slabs) {
+  int tile = kVTok;
+  while (tile > kVTokMin && (tokens + tile - 1) / tile * slabs < kConvBlocks) tile /= 2;
+  return tile;
+}
 
 // FRONT: fused front end (q/k normalised into q_out/k_out, v into v_out, history
 // from the pool); otherwise the plain packed conv into conv.out.
@@ -233,8 +248,8 @@ __global__ __launch_bounds__(256) void conv_vec_kernel(FrontParams fp) {
   constexpr int S = W - 1;
   const int64_t ch0 = (static_cast<int64_t>(blockIdx.y) * 256 + threadIdx.x) * 8;
   const bool active = ch0 < p.C;
-  const int64_t t0 = static_cast<int64_t>(blockIdx.x) * kVTok;
-  const int64_t t1 = tile_end(p.cu, p.cu_is64, p.N, p.T, t0, kVTok);
+  const int64_t t0 = static_cast<int64_t>(blockIdx.x) * fp.tile;
+  const int64_t t1 = tile_end(p.cu, p.cu_is64, p.N, p.T, t0, fp.tile);
   if (t0 >= t1) return;  // whole block: padding rows only
   const int64_t key_dim = FRONT ? fp.H * DK : 0;
   float w[W][8], bias[8];
@@ -437,14 +452,16 @@ __global__ __launch_bounds__(256) void conv_vec_kernel(FrontParams fp) {
 
 // Launch the vectorised kernel when the layout allows it; returns -1 if not.
 template <class T, bool FRONT>
-int launch_vec(const FrontParams& fp, int dk, hipStream_t s) {
+int launch_vec(FrontParams fp, int dk, hipStream_t s) {
   const ConvParams& p = fp.conv;
   const bool aligned = p.xc == 1 && p.xr % 8 == 0 && p.C % 8 == 0 &&
                        (reinterpret_cast<uintptr_t>(p.x) & 15) == 0 && (reinterpret_cast<uintptr_t>(p.w) & 15) == 0 &&
                        (!p.bias || (reinterpret_cast<uintptr_t>(p.bias) & 15) == 0) &&
                        (FRONT || (reinterpret_cast<uintptr_t>(p.out) & 15) == 0) && p.W >= 2 && p.W <= 4;
   if (!aligned) return -1;
-  dim3 grid(static_cast<unsigned>((p.T + kVTok - 1) / kVTok), static_cast<unsigned>((p.C / 8 + 255) / 256));
+  const int64_t slabs = (p.C / 8 + 255) / 256;
+  fp.tile = conv_tile(p.T, slabs);
+  dim3 grid(static_cast<unsigned>((p.T + fp.tile - 1) / fp.tile), static_cast<unsigned>(slabs));
   auto go = [&](auto Wc, auto DKc) {
     constexpr int Wv = decltype(Wc)::value, DKv = decltype(DKc)::value;
     hipLaunchKernelGGL((conv_vec_kernel<T, Wv, DKv, FRONT>), grid, dim3(256), 0, s, fp);
