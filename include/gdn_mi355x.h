@@ -169,6 +169,41 @@ int gdn_chunk_gated_delta_rule_logged(const void* q, const void* k, const void* 
                                       void* out, float scale, void* stream);
 
 /*
+ * The chunked rule with a workspace, for few sequences: with at least
+ * gdn_chunk_workspace_bytes(...) bytes (16-byte aligned) the state-independent
+ * parts of every 64-token chunk are formed in one parallel launch and kept
+ * there, and a second launch runs the recurrence over them.  Same results bit
+ * for bit as gdn_chunk_gated_delta_rule and gdn_chunk_gated_delta_rule_logged;
+ * with a null or smaller workspace they are those entry points.  The workspace
+ * is scratch: its contents need not outlive the stream's work.
+ */
+int gdn_chunk_gated_delta_rule_ws(const void* q, const void* k, const void* v, int io_dtype, const float* g,
+                                  const float* beta, const void* cu_seqlens, int cu_dtype, int64_t num_seqs,
+                                  int64_t total_tokens, int64_t H, int64_t HV, int64_t dk, int64_t dv,
+                                  void* state, int state_dtype, int64_t slot_stride, int64_t layer_stride,
+                                  int64_t head_stride, int64_t layer, const void* read_slots, int read_dtype,
+                                  const void* chunk_write_slots, int chunk_write_dtype,
+                                  const void* final_write_slots, int final_write_dtype, int64_t chunk_size,
+                                  const void* frames, int frames_dtype, int64_t table_rows, int64_t frames_per_slot,
+                                  int64_t frame_bytes, int64_t head_bytes, int64_t num_frames, void* out, void* v_new,
+                                  float scale, void* workspace, int64_t workspace_bytes, void* stream);
+int gdn_chunk_gated_delta_rule_logged_ws(const void* q, const void* k, const void* v, int io_dtype, const float* g,
+                                         const float* beta, const void* cu_seqlens, int cu_dtype, int64_t num_seqs,
+                                         int64_t total_tokens, int64_t H, int64_t HV, int64_t dk, int64_t dv,
+                                         void* state, int state_dtype, int64_t layer, const void* read_slots,
+                                         int read_dtype, const void* chunk_write_slots, int chunk_write_dtype,
+                                         const void* final_write_slots, int final_write_dtype, int64_t chunk_size,
+                                         const void* frames, int frames_dtype, int64_t table_rows,
+                                         int64_t frames_per_slot, int64_t frame_bytes, int64_t head_bytes,
+                                         int64_t num_frames, const void* log_slots, int log_dtype,
+                                         const void* token_offsets, int offsets_dtype, int64_t key_heads,
+                                         int64_t num_layers, int64_t page_size, void* out, float scale,
+                                         void* workspace, int64_t workspace_bytes, void* stream);
+/* Workspace with which the chunked rule is faster, or 0 where it is not (logging: the _logged form). */
+int64_t gdn_chunk_workspace_bytes(int64_t num_seqs, int64_t total_tokens, int64_t H, int64_t HV, int64_t dk,
+                                  int64_t dv, int logging);
+
+/*
  * LogState token log of the chunked prefill: replaces the log stores of
  * kernel/linear_attention/state_io.py:83-126 (_store_chunk_log, called from
  * vendor/fla/chunk_delta_h.py:183-192 when a ChunkLogIO is given), with the
@@ -405,6 +440,27 @@ int gdn_prefill_fused(const void* q, const void* k, const void* mixed, int64_t r
                       int chunk_write_dtype, const void* final_write_slots, int final_write_dtype,
                       const void* snapshot_rows, int rows_dtype, const void* snapshot_slots, int slots_dtype,
                       int64_t snapshot_count, void* out, float scale, void* stream);
+
+/*
+ * The same prefill for few sequences, in one call: gdn_prefill_frontend, the
+ * chunked rule with a workspace and gdn_conv_snapshots, with the front end's
+ * outputs in the workspace too (at least gdn_prefill_workspace_bytes(...), 0
+ * where gdn_prefill_qk + gdn_prefill_fused are faster).  Arguments as there;
+ * same results bit for bit.
+ */
+int gdn_prefill_split(const void* mixed, int64_t row_stride, int io_dtype, const void* weight, int kernel_width,
+                      const void* cu_seqlens, int cu_dtype, int64_t num_seqs, int64_t total_tokens, int64_t H,
+                      int64_t HV, int64_t dk, int64_t dv, void* conv_state, int64_t conv_slot_stride,
+                      int64_t conv_layer_stride, const void* gate, int64_t gate_row_stride, int64_t gate_head_stride,
+                      int gate_dtype, const void* beta, int64_t beta_row_stride, int64_t beta_head_stride,
+                      int beta_dtype, const void* A_log, int a_dtype, const void* dt_bias, int dt_dtype, void* state,
+                      int state_dtype, int64_t slot_stride, int64_t layer_stride, int64_t head_stride, int64_t layer,
+                      const void* baseline_slots, int baseline_dtype, const void* chunk_write_slots,
+                      int chunk_write_dtype, const void* snapshot_rows, int snapshot_rows_dtype,
+                      const void* snapshot_slots, int snapshot_slots_dtype, int64_t snapshot_count, void* out,
+                      float scale, void* workspace, int64_t workspace_bytes, void* stream);
+int64_t gdn_prefill_workspace_bytes(int64_t num_seqs, int64_t total_tokens, int64_t H, int64_t HV, int64_t dk,
+                                    int64_t dv);
 
 /*
  * gdn_conv_snapshots: for each i < count with slots[i] >= 0, conv_state[slots[i],

@@ -22,7 +22,7 @@ I32 = ctypes.c_int
 F32 = ctypes.c_float
 PI64 = ctypes.POINTER(ctypes.c_int64)
 
-# name -> argtypes (restype is always int)
+# name -> argtypes (restype int; int64 for the *_workspace_bytes queries)
 SIGNATURES = {
     "gdn_packed_causal_conv1d": [P, I64, I64, I32, P, P, P, P, I32, I64, I64, I64, I32, P, P, I64, I64, I64,
                                  P, I32, P, I32, I64, I64, F32, F32, F32, P],
@@ -35,6 +35,17 @@ SIGNATURES = {
                        P, I64, I64, I32, P, I64, I64, I32, P, I32, P, I32, P, P, P],
     "gdn_prefill_fused": [P, P, P, I64, I32, P, I32, P, I32, I64, I64, I64, I64, I64, I64, P, I64, I64, P, P, P, I32,
                           I64, I64, I64, I64, P, I32, P, I32, P, I32, P, I32, P, I32, I64, P, F32, P],
+    "gdn_prefill_split": [P, I64, I32, P, I32, P, I32, I64, I64, I64, I64, I64, I64, P, I64, I64, P, I64, I64, I32, P,
+                          I64, I64, I32, P, I32, P, I32, P, I32, I64, I64, I64, I64, P, I32, P, I32, P, I32, P, I32,
+                          I64, P, F32, P, I64, P],
+    "gdn_prefill_workspace_bytes": [I64, I64, I64, I64, I64, I64],
+    "gdn_chunk_workspace_bytes": [I64, I64, I64, I64, I64, I64, I32],
+    "gdn_chunk_gated_delta_rule_ws": [P, P, P, I32, P, P, P, I32, I64, I64, I64, I64, I64, I64, P, I32, I64, I64, I64,
+                                      I64, P, I32, P, I32, P, I32, I64, P, I32, I64, I64, I64, I64, I64, P, P, F32, P,
+                                      I64, P],
+    "gdn_chunk_gated_delta_rule_logged_ws": [P, P, P, I32, P, P, P, I32, I64, I64, I64, I64, I64, I64, P, I32, I64, P,
+                                             I32, P, I32, P, I32, I64, P, I32, I64, I64, I64, I64, I64, P, I32, P,
+                                             I32, I64, I64, I64, P, F32, P, I64, P],
     "gdn_metadata_copy": [P, P, PI64, PI64, PI64, P, I32, P],
     "gdn_metadata_pad": [P, P, PI64, PI64, PI64, PI64, P, I32, P],
     "gdn_rms_norm_gated": [P, I32, I64, I64, P, I32, I64, I64, I64, I64, P, I32, F32, P, P],
@@ -100,7 +111,7 @@ def lib() -> ctypes.CDLL:
         for name, args in SIGNATURES.items():
             fn = getattr(handle, name)
             fn.argtypes = args
-            fn.restype = ctypes.c_int
+            fn.restype = I64 if name.endswith("_workspace_bytes") else ctypes.c_int
         handle.gdn_last_error.argtypes = []
         handle.gdn_last_error.restype = ctypes.c_char_p
         handle.gdn_abi_version.argtypes = []
@@ -119,6 +130,13 @@ def call(name: str, *args) -> None:
         if rc == 2:
             raise NotImplementedError(f"{name}: {msg}")
         raise RuntimeError(f"{name} failed ({rc}): {msg}")
+
+
+def workspace(name: str, device, *sizes) -> tuple[torch.Tensor | None, int]:
+    """The workspace the ``name`` query asks for (scratch of the current
+    stream's work), and its bytes: ``(None, 0)`` where none is used."""
+    n = getattr(lib(), name)(*sizes)
+    return (torch.empty(n, dtype=torch.uint8, device=device), n) if n else (None, 0)
 
 
 def dtype_code(dtype: torch.dtype) -> int:

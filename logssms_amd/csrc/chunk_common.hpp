@@ -95,5 +95,13 @@ int launch_chunk_chain(const ChunkParams& p, int64_t dk, int io_dtype, int state
 int launch_chunk_chain_fused(const ChunkParams& p, int64_t dk, int io_dtype, int state_dtype, int64_t groups,
                              hipStream_t stream);
 
+// Two-launch form for few sequences (chunk_scan.hip): records of every chunk
+// in `workspace` (chunk_scan_workspace bytes), then the recurrence; d_k in
+// {32, 64, 128}, d_v a multiple of 16, the same results bit for bit.
+// chunk_scan_preferred: whether it is the faster form.
+int64_t chunk_scan_workspace(int64_t num_seqs, int64_t total_tokens, int64_t HV, int64_t dv, bool logging);
+bool chunk_scan_preferred(int64_t num_seqs, int64_t total_tokens, int64_t HV, int64_t dv);
+int launch_chunk_scan(const ChunkParams& p, int64_t dk, int io_dtype, int state_dtype, void* workspace,
+                      hipStream_t stream);
 
 }  // namespace gdn

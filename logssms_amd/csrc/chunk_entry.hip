@@ -4,7 +4,7 @@
 // layout validation and the launch of the register-chain kernel
 // (chunk_chain.hip), which covers d_k in {32, 64, 128} and d_v = 32 or a
 // multiple of 64.
-#include "chunk_common.hpp"
+#include "chunk_tile.hpp"
 
 namespace gdn {
 
@@ -41,6 +41,10 @@ int set_frame_layout(ChunkParams& p, int64_t dk, int state_dtype, const void* fr
 }
 
 namespace {
+// Largest workspace asked for (46,000 tokens of a prefill at 16 / 32 heads of
+// 128): longer calls keep to the one-launch kernel and its smaller footprint.
+constexpr int64_t kMaxWorkspace = int64_t{1} << 30;
+
 // The token log arguments of gdn_chunk_gated_delta_rule_logged.
 struct LogArgs {
   const void* slots;
@@ -57,7 +61,7 @@ int chunk_entry(const void* q, const void* k, const void* v, int io_dtype, const
                 const void* chunk_write_slots, int chunk_write_dtype, const void* final_write_slots,
                 int final_write_dtype, int64_t chunk_size, const void* frames, int frames_dtype, int64_t table_rows,
                 int64_t frames_per_slot, int64_t frame_bytes, int64_t head_bytes, int64_t num_frames, void* out,
-                void* v_new, float scale, const LogArgs* log, void* stream) {
+                void* v_new, float scale, const LogArgs* log, void* workspace, int64_t workspace_bytes, void* stream) {
   GDN_REQUIRE(num_seqs >= 0 && total_tokens >= 0 && H > 0 && HV > 0 && HV % H == 0 && layer >= 0,
               "gdn_chunk_gated_delta_rule: bad sizes");
   GDN_REQUIRE(chunk_size == 16 || chunk_size == 32 || chunk_size == 64,
@@ -116,7 +120,10 @@ int chunk_entry(const void* q, const void* k, const void* v, int io_dtype, const
   }
   p.nvs = static_cast<int>((dv + 63) / 64);
   p.members = static_cast<int>((HV / H) * p.nvs);
-  const int rc = launch_chunk_chain(p, dk, io_dtype, state_dtype, num_seqs * H, static_cast<hipStream_t>(stream));
+  const bool scan = workspace &&
+                    workspace_bytes >= chunk_scan_workspace(num_seqs, total_tokens, HV, dv, log != nullptr);
+  const int rc = scan ? launch_chunk_scan(p, dk, io_dtype, state_dtype, workspace, static_cast<hipStream_t>(stream))
+                      : launch_chunk_chain(p, dk, io_dtype, state_dtype, num_seqs * H, static_cast<hipStream_t>(stream));
   if (rc == GDN_ERR_UNSUPPORTED)
     set_error("gdn_chunk_gated_delta_rule: unsupported io/state dtypes %d/%d (16-bit io, fp32 or io-typed state)",
               io_dtype, state_dtype);
@@ -139,7 +146,43 @@ extern "C" int gdn_chunk_gated_delta_rule(const void* q, const void* k, const vo
                           state, state_dtype, slot_stride, layer_stride, head_stride, layer, read_slots, read_dtype,
                           chunk_write_slots, chunk_write_dtype, final_write_slots, final_write_dtype, chunk_size, frames,
                           frames_dtype, table_rows, frames_per_slot, frame_bytes, head_bytes, num_frames, out, v_new,
-                          scale, nullptr, stream);
+                          scale, nullptr, nullptr, 0, stream);
+}
+
+extern "C" int gdn_chunk_gated_delta_rule_ws(const void* q, const void* k, const void* v, int io_dtype, const float* g,
+                                             const float* beta, const void* cu_seqlens, int cu_dtype, int64_t num_seqs,
+                                             int64_t total_tokens, int64_t H, int64_t HV, int64_t dk, int64_t dv,
+                                             void* state, int state_dtype, int64_t slot_stride, int64_t layer_stride,
+                                             int64_t head_stride, int64_t layer, const void* read_slots, int read_dtype,
+                                             const void* chunk_write_slots, int chunk_write_dtype,
+                                             const void* final_write_slots, int final_write_dtype, int64_t chunk_size,
+                                             const void* frames, int frames_dtype, int64_t table_rows,
+                                             int64_t frames_per_slot, int64_t frame_bytes, int64_t head_bytes,
+                                             int64_t num_frames, void* out, void* v_new, float scale, void* workspace,
+                                             int64_t workspace_bytes, void* stream) {
+  return gdn::chunk_entry(q, k, v, io_dtype, g, beta, cu_seqlens, cu_dtype, num_seqs, total_tokens, H, HV, dk, dv,
+                          state, state_dtype, slot_stride, layer_stride, head_stride, layer, read_slots, read_dtype,
+                          chunk_write_slots, chunk_write_dtype, final_write_slots, final_write_dtype, chunk_size, frames,
+                          frames_dtype, table_rows, frames_per_slot, frame_bytes, head_bytes, num_frames, out, v_new,
+                          scale, nullptr, workspace, workspace_bytes, stream);
+}
+
+extern "C" int gdn_chunk_gated_delta_rule_logged_ws(
+    const void* q, const void* k, const void* v, int io_dtype, const float* g, const float* beta,
+    const void* cu_seqlens, int cu_dtype, int64_t num_seqs, int64_t total_tokens, int64_t H, int64_t HV, int64_t dk,
+    int64_t dv, void* state, int state_dtype, int64_t layer, const void* read_slots, int read_dtype,
+    const void* chunk_write_slots, int chunk_write_dtype, const void* final_write_slots, int final_write_dtype,
+    int64_t chunk_size, const void* frames, int frames_dtype, int64_t table_rows, int64_t frames_per_slot,
+    int64_t frame_bytes, int64_t head_bytes, int64_t num_frames, const void* log_slots, int log_dtype,
+    const void* token_offsets, int offsets_dtype, int64_t key_heads, int64_t num_layers, int64_t page_size, void* out,
+    float scale, void* workspace, int64_t workspace_bytes, void* stream) {
+  GDN_REQUIRE(frames, "gdn_chunk_gated_delta_rule_logged: the token log lives in frame storage");
+  const gdn::LogArgs log{log_slots, log_dtype, token_offsets, offsets_dtype, key_heads, num_layers, page_size};
+  return gdn::chunk_entry(q, k, v, io_dtype, g, beta, cu_seqlens, cu_dtype, num_seqs, total_tokens, H, HV, dk, dv,
+                          state, state_dtype, 0, 0, 0, layer, read_slots, read_dtype, chunk_write_slots,
+                          chunk_write_dtype, final_write_slots, final_write_dtype, chunk_size, frames, frames_dtype,
+                          table_rows, frames_per_slot, frame_bytes, head_bytes, num_frames, out, nullptr, scale, &log,
+                          workspace, workspace_bytes, stream);
 }
 
 extern "C" int gdn_chunk_gated_delta_rule_logged(
@@ -151,11 +194,83 @@ extern "C" int gdn_chunk_gated_delta_rule_logged(
     int64_t frame_bytes, int64_t head_bytes, int64_t num_frames, const void* log_slots, int log_dtype,
     const void* token_offsets, int offsets_dtype, int64_t key_heads, int64_t num_layers, int64_t page_size, void* out,
     float scale, void* stream) {
-  GDN_REQUIRE(frames, "gdn_chunk_gated_delta_rule_logged: the token log lives in frame storage");
-  const gdn::LogArgs log{log_slots, log_dtype, token_offsets, offsets_dtype, key_heads, num_layers, page_size};
-  return gdn::chunk_entry(q, k, v, io_dtype, g, beta, cu_seqlens, cu_dtype, num_seqs, total_tokens, H, HV, dk, dv,
-                          state, state_dtype, 0, 0, 0, layer, read_slots, read_dtype, chunk_write_slots,
-                          chunk_write_dtype, final_write_slots, final_write_dtype, chunk_size, frames, frames_dtype,
-                          table_rows, frames_per_slot, frame_bytes, head_bytes, num_frames, out, nullptr, scale, &log,
-                          stream);
+  return gdn_chunk_gated_delta_rule_logged_ws(
+      q, k, v, io_dtype, g, beta, cu_seqlens, cu_dtype, num_seqs, total_tokens, H, HV, dk, dv, state, state_dtype,
+      layer, read_slots, read_dtype, chunk_write_slots, chunk_write_dtype, final_write_slots, final_write_dtype,
+      chunk_size, frames, frames_dtype, table_rows, frames_per_slot, frame_bytes, head_bytes, num_frames, log_slots,
+      log_dtype, token_offsets, offsets_dtype, key_heads, num_layers, page_size, out, scale, nullptr, 0, stream);
+}
+
+extern "C" int64_t gdn_chunk_workspace_bytes(int64_t num_seqs, int64_t total_tokens, int64_t H, int64_t HV,
+                                             int64_t dk, int64_t dv, int logging) {
+  if (num_seqs < 1 || total_tokens < 1 || H < 1 || HV < 1 || dk < 1 || dv < 1) return 0;
+  const int64_t bytes = gdn::chunk_scan_workspace(num_seqs, total_tokens, HV, dv, logging != 0);
+  return gdn::chunk_scan_preferred(num_seqs, total_tokens, HV, dv) && bytes <= gdn::kMaxWorkspace ? bytes : 0;
+}
+
+// The split prefill: front end (q, k, v and gates in HBM), chunk records and
+// recurrence, conv windows.  Staging carved from the caller's workspace.
+namespace gdn {
+namespace {
+struct SplitStaging {
+  int64_t q, k, v, g, b, rules, bytes;
+};
+SplitStaging split_staging(int64_t num_seqs, int64_t T, int64_t H, int64_t HV, int64_t dk, int64_t dv) {
+  auto align = [](int64_t x) { return (x + 255) / 256 * 256; };
+  SplitStaging s{};
+  s.k = align(T * H * dk * 2);
+  s.v = 2 * s.k;
+  s.g = s.v + align(T * HV * dv * 2);
+  s.b = s.g + align(T * HV * 4);
+  s.rules = s.b + align(T * HV * 4);
+  s.bytes = s.rules + chunk_scan_workspace(num_seqs, T, HV, dv, false);
+  return s;
+}
+}  // namespace
+}  // namespace gdn
+
+extern "C" int64_t gdn_prefill_workspace_bytes(int64_t num_seqs, int64_t total_tokens, int64_t H, int64_t HV,
+                                               int64_t dk, int64_t dv) {
+  if (num_seqs < 1 || total_tokens < 1 || H < 1 || HV < 1 || dk < 1 || dv < 1) return 0;
+  const int64_t bytes = gdn::split_staging(num_seqs, total_tokens, H, HV, dk, dv).bytes;
+  return gdn::chunk_scan_preferred(num_seqs, total_tokens, HV, dv) && bytes <= gdn::kMaxWorkspace ? bytes : 0;
+}
+
+extern "C" int gdn_prefill_split(const void* mixed, int64_t row_stride, int io_dtype, const void* weight,
+                                 int kernel_width, const void* cu_seqlens, int cu_dtype, int64_t num_seqs,
+                                 int64_t total_tokens, int64_t H, int64_t HV, int64_t dk, int64_t dv, void* conv_state,
+                                 int64_t conv_slot_stride, int64_t conv_layer_stride, const void* gate,
+                                 int64_t gate_row_stride, int64_t gate_head_stride, int gate_dtype, const void* beta,
+                                 int64_t beta_row_stride, int64_t beta_head_stride, int beta_dtype, const void* A_log,
+                                 int a_dtype, const void* dt_bias, int dt_dtype, void* state, int state_dtype,
+                                 int64_t slot_stride, int64_t layer_stride, int64_t head_stride, int64_t layer,
+                                 const void* baseline_slots, int baseline_dtype, const void* chunk_write_slots,
+                                 int chunk_write_dtype, const void* snapshot_rows, int snapshot_rows_dtype,
+                                 const void* snapshot_slots, int snapshot_slots_dtype, int64_t snapshot_count,
+                                 void* out, float scale, void* workspace, int64_t workspace_bytes, void* stream) {
+  using namespace gdn;
+  GDN_REQUIRE(num_seqs >= 1 && total_tokens >= 1 && H > 0 && HV > 0 && HV % H == 0 && dk > 0 && dv > 0,
+              "gdn_prefill_split: bad sizes");
+  const SplitStaging at = split_staging(num_seqs, total_tokens, H, HV, dk, dv);
+  GDN_REQUIRE(workspace && workspace_bytes >= at.bytes && aligned16(workspace),
+              "gdn_prefill_split: %lld bytes of 16-byte aligned workspace needed", (long long)at.bytes);
+  char* w = static_cast<char*>(workspace);
+  float* g = reinterpret_cast<float*>(w + at.g);
+  float* b = reinterpret_cast<float*>(w + at.b);
+  int rc = gdn_prefill_frontend(mixed, row_stride, 1, io_dtype, weight, nullptr, kernel_width, cu_seqlens, cu_dtype,
+                                num_seqs, total_tokens, H, HV, dk, dv, conv_state, conv_slot_stride, conv_layer_stride,
+                                layer, baseline_slots, baseline_dtype, gate, gate_row_stride, gate_head_stride,
+                                gate_dtype, beta, beta_row_stride, beta_head_stride, beta_dtype, A_log, a_dtype,
+                                dt_bias, dt_dtype, w + at.q, w + at.k, w + at.v, g, b, stream);
+  if (rc != GDN_OK) return rc;
+  rc = gdn_chunk_gated_delta_rule_ws(w + at.q, w + at.k, w + at.v, io_dtype, g, b, cu_seqlens, cu_dtype, num_seqs,
+                                     total_tokens, H, HV, dk, dv, state, state_dtype, slot_stride, layer_stride,
+                                     head_stride, layer, baseline_slots, baseline_dtype, chunk_write_slots,
+                                     chunk_write_dtype, nullptr, 0, kC, nullptr, 0, 0, 0, 0, 0, 0, out, nullptr, scale,
+                                     w + at.rules, at.bytes - at.rules, stream);
+  if (rc != GDN_OK || snapshot_count == 0) return rc;
+  return gdn_conv_snapshots(mixed, row_stride, io_dtype, cu_seqlens, cu_dtype, num_seqs, total_tokens,
+                            2 * H * dk + HV * dv, kernel_width, conv_state, conv_slot_stride, conv_layer_stride, layer,
+                            baseline_slots, baseline_dtype, snapshot_rows, snapshot_rows_dtype, snapshot_slots,
+                            snapshot_slots_dtype, snapshot_count, stream);
 }

@@ -66,7 +66,7 @@ extern "C" int gdn_stamps_simds(void* out_dev, int blocks, void* stream) {
 def instrument(src):
     """The stamped source: STAMP around each loop barrier (the kernel's own
     `wave` and `lane`: wave w runs on the SIMD HW_ID reports)."""
-    anchor = "constexpr int kC = 64;"
+    anchor = "constexpr int kThreads = 768;"
     if src.count(anchor) != 1:
         raise SystemExit("chunk_stamps: chunk_chain.hip has no unique '%s'" % anchor)
     out = src.replace(anchor, MACRO + anchor, 1)

@@ -145,6 +145,10 @@ def prefill_fused(mixed_qkv, gate, beta, conv_weight, A_log, dt_bias, config, co
     assert out.shape == (T, config.num_v_heads, config.head_v_dim) and out.is_contiguous()
     A_log = A_log.contiguous()
     dt_bias = dt_bias.contiguous()
+    if T and chunk_events is None and _prefill_split(mixed_qkv, gate, beta, weight, A_log, dt_bias, config, conv_state,
+                                                     recurrent_state, cu_seqlens, baseline_slots, chunk_write_slots,
+                                                     snapshot_rows, snapshot_slots, out):
+        return out
     # q, k as the chunk kernel's f16 MFMA operands; prepared gates
     q = torch.empty(T, config.num_k_heads, config.head_k_dim, device=mixed_qkv.device, dtype=torch.float16)
     k = torch.empty_like(q)
@@ -171,6 +175,35 @@ def prefill_fused(mixed_qkv, gate, beta, conv_weight, A_log, dt_bias, config, co
     if chunk_events is not None:
         chunk_events[1].record()
     return out
+
+
+def _prefill_split(mixed_qkv, gate, beta, weight, A_log, dt_bias, config, conv_state, recurrent_state, cu_seqlens,
+                   baseline_slots, chunk_write_slots, snapshot_rows, snapshot_slots, out) -> bool:
+    """``prefill_fused`` for few sequences (``gdn_prefill_split``: the
+    recurrence kept apart from the parallel work of the chunks); False, with
+    nothing launched, where the fused launches are the faster ones."""
+    T, N = mixed_qkv.shape[0], len(cu_seqlens) - 1
+    ws, ws_bytes = _lib.workspace("gdn_prefill_workspace_bytes", mixed_qkv.device, N, T, config.num_k_heads,
+                                  config.num_v_heads, config.head_k_dim, config.head_v_dim)
+    if ws is None:
+        return False
+    count = snapshot_rows.numel()
+    assert not count or (snapshot_rows.is_contiguous() and snapshot_slots.is_contiguous())
+    _lib.call(
+        "gdn_prefill_split", mixed_qkv.data_ptr(), mixed_qkv.stride(0), _lib.dtype_code(mixed_qkv.dtype),
+        weight.data_ptr(), 4, cu_seqlens.data_ptr(), _lib.index_code(cu_seqlens), N, T, config.num_k_heads,
+        config.num_v_heads, config.head_k_dim, config.head_v_dim, conv_state.data_ptr(), conv_state.stride(0),
+        conv_state.stride(1), gate.data_ptr(), gate.stride(0), gate.stride(1), _lib.dtype_code(gate.dtype),
+        beta.data_ptr(), beta.stride(0), beta.stride(1), _lib.dtype_code(beta.dtype),
+        A_log.data_ptr(), _lib.dtype_code(A_log.dtype), dt_bias.data_ptr(), _lib.dtype_code(dt_bias.dtype),
+        recurrent_state.data_ptr(), _lib.dtype_code(recurrent_state.dtype), recurrent_state.stride(0),
+        recurrent_state.stride(1), recurrent_state.stride(2), config.layer_idx,
+        baseline_slots.data_ptr(), _lib.index_code(baseline_slots), chunk_write_slots.data_ptr(),
+        _lib.index_code(chunk_write_slots), snapshot_rows.data_ptr() if count else None,
+        _lib.index_code(snapshot_rows) if count else 0, snapshot_slots.data_ptr() if count else None,
+        _lib.index_code(snapshot_slots) if count else 0, count, out.data_ptr(), float(config.head_k_dim) ** -0.5,
+        ws.data_ptr(), ws_bytes, _lib.stream_of(mixed_qkv))
+    return True
 
 
 def prefill_fused_noalloc(mixed_qkv, gate, beta, conv_weight, A_log, dt_bias, config, conv_state, recurrent_state,

@@ -108,10 +108,13 @@ def chunk_gated_delta_rule_to_cache(
     # v' straight into the log when the caller does not want v_new back
     direct_log = (log_io is not None and not return_v_new and state_io.frame_bytes % (2 * min(dv, 64)) == 0)
     v_new = torch.empty_like(value) if (return_v_new or (log_io is not None and not direct_log)) else None
+    if T:  # few sequences: scratch for the two-launch form (kept by the allocator's stream order)
+        ws, ws_bytes = _lib.workspace("gdn_chunk_workspace_bytes", query.device, len(cu_seqlens) - 1, T, H, HV, dk, dv,
+                                      int(direct_log))
     if T and direct_log:
         fw = state_io.final_write_slots
         _lib.call(
-            "gdn_chunk_gated_delta_rule_logged",
+            "gdn_chunk_gated_delta_rule_logged_ws",
             query.data_ptr(), key.data_ptr(), value.data_ptr(), _lib.dtype_code(value.dtype),
             gate.data_ptr(), beta.data_ptr(), cu_seqlens.data_ptr(), _lib.index_code(cu_seqlens),
             len(cu_seqlens) - 1, T, H, HV, dk, dv,
@@ -123,12 +126,12 @@ def chunk_gated_delta_rule_to_cache(
             log_io.slots.data_ptr(), _lib.index_code(log_io.slots),
             log_io.token_offsets.data_ptr(), _lib.index_code(log_io.token_offsets),
             log_io.num_key_heads, state_io.num_layers, log_io.page_size,
-            o.data_ptr(), float(dk) ** -0.5, _lib.stream_of(query),
+            o.data_ptr(), float(dk) ** -0.5, _lib.ptr(ws), ws_bytes, _lib.stream_of(query),
         )
     elif T:
         fw = state_io.final_write_slots
         _lib.call(
-            "gdn_chunk_gated_delta_rule",
+            "gdn_chunk_gated_delta_rule_ws",
             query.data_ptr(), key.data_ptr(), value.data_ptr(), _lib.dtype_code(value.dtype),
             gate.data_ptr(), beta.data_ptr(), cu_seqlens.data_ptr(), _lib.index_code(cu_seqlens),
             len(cu_seqlens) - 1, T, H, HV, dk, dv,
@@ -137,7 +140,7 @@ def chunk_gated_delta_rule_to_cache(
             state_io.chunk_write_slots.data_ptr(), _lib.index_code(state_io.chunk_write_slots),
             _lib.ptr(fw), _lib.index_code(fw) if fw is not None else 0, chunk_size,
             _lib.ptr(frame_args[0]), *frame_args[1:],
-            o.data_ptr(), _lib.ptr(v_new), float(dk) ** -0.5, _lib.stream_of(query),
+            o.data_ptr(), _lib.ptr(v_new), float(dk) ** -0.5, _lib.ptr(ws), ws_bytes, _lib.stream_of(query),
         )
     if T and log_io is not None:
         log_gate = log_io.gate.float().contiguous()
