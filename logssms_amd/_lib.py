@@ -3,7 +3,8 @@ declared in ``include/gdn_mi355x.h``).
 
 There is no fallback: if the library is missing or a call fails, a
 ``RuntimeError`` is raised.  Tensors are passed as raw device pointers; the
-launch goes on torch's current stream of the tensor's device.
+launch goes on torch's current stream of the tensor's device.  The hot entry
+points are called through ``_host.so``, the others through ctypes.
 """
 
 from __future__ import annotations
@@ -122,9 +123,34 @@ def lib() -> ctypes.CDLL:
     return _lib
 
 
+_host = None
+
+
+def host():
+    """``logssms_amd._host`` (csrc/host.cpp), the host side of the per-layer
+    calls, loaded once; raise if it has not been built."""
+    global _host
+    if _host is None:
+        lib()
+        try:
+            from . import _host as module
+        except ImportError as err:
+            raise RuntimeError(f"logssms_amd/_host.so cannot be loaded ({err}): build it with `make -C logssms_amd/csrc`"
+                               ) from err
+        _host = module
+    return _host
+
+
+def entry(name: str):
+    """The callable of a C-ABI function: its typed entry in ``_host`` where
+    there is one, else ctypes."""
+    fn = getattr(host(), name, None)
+    return getattr(lib(), name) if fn is None else fn
+
+
 def call(name: str, *args) -> None:
     """Invoke ``name`` and raise ``RuntimeError`` with the library's message on failure."""
-    rc = getattr(lib(), name)(*args)
+    rc = entry(name)(*args)
     if rc != 0:
         msg = lib().gdn_last_error().decode(errors="replace")
         if rc == 2:
@@ -135,7 +161,7 @@ def call(name: str, *args) -> None:
 def workspace(name: str, device, *sizes) -> tuple[torch.Tensor | None, int]:
     """The workspace the ``name`` query asks for (scratch of the current
     stream's work), and its bytes: ``(None, 0)`` where none is used."""
-    n = getattr(lib(), name)(*sizes)
+    n = entry(name)(*sizes)
     return (torch.empty(n, dtype=torch.uint8, device=device), n) if n else (None, 0)
 
 
@@ -161,7 +187,7 @@ def ptr(t: torch.Tensor | None) -> int | None:
 def stream_of(t: torch.Tensor) -> int:
     if not t.is_cuda:
         raise RuntimeError("libgdn_mi355x kernels need tensors on a ROCm device")
-    return torch.cuda.current_stream(t.device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
 def i64_array(values):

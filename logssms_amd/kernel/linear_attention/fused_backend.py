@@ -270,26 +270,13 @@ def prefill_chunk_fused(q, k, g, b, mixed_qkv, weight, config, conv_state, recur
 
 
 def _fused(mixed, row_index, gate, beta, conv_weight, A_log, dt_bias, config, conv_state, recurrent_state,
-           read_slots, write_slots, batch, steps, write_b, write_t, out):
-    weight = conv_weight.contiguous()
-    A_log = A_log.contiguous()
-    dt_bias = dt_bias.contiguous()
-    _lib.call(
-        "gdn_fused_conv_recurrent",
-        mixed.data_ptr(), mixed.stride(0), mixed.stride(1), _lib.dtype_code(mixed.dtype),
-        _lib.ptr(row_index), _lib.index_code(row_index) if row_index is not None else 0,
-        weight.data_ptr(), None, config.state_len + 1,
-        gate.data_ptr(), gate.stride(0), gate.stride(1), _lib.dtype_code(gate.dtype),
-        beta.data_ptr(), beta.stride(0), beta.stride(1), _lib.dtype_code(beta.dtype),
-        A_log.data_ptr(), _lib.dtype_code(A_log.dtype), dt_bias.data_ptr(), _lib.dtype_code(dt_bias.dtype),
-        batch, steps, config.num_k_heads, config.num_v_heads, config.head_k_dim, config.head_v_dim,
-        conv_state.data_ptr(), conv_state.stride(0), conv_state.stride(1),
-        recurrent_state.data_ptr(), _lib.dtype_code(recurrent_state.dtype), recurrent_state.stride(0),
-        recurrent_state.stride(1), recurrent_state.stride(2), config.layer_idx,
-        read_slots.data_ptr(), read_slots.stride(0), _lib.index_code(read_slots),
-        write_slots.data_ptr(), write_b, write_t, _lib.index_code(write_slots),
-        out.data_ptr(), float(config.head_k_dim) ** -0.5, _lib.stream_of(mixed),
-    )
+           read_slots, write_slots, out):
+    """One ``gdn_fused_conv_recurrent`` call, checked and issued natively
+    (``_host.conv_recurrent``); write slots [B] for decode, [B, T] for verify."""
+    return _lib.host().conv_recurrent(
+        mixed, row_index, gate, beta, conv_weight, A_log, dt_bias, conv_state, recurrent_state, read_slots, write_slots,
+        out, config.num_k_heads, config.num_v_heads, config.head_k_dim, config.head_v_dim, config.conv_dim,
+        config.state_len, config.layer_idx)
 
 
 # limits of gdn_fused_conv_recurrent: drafts per launch, v-heads per key head
@@ -327,6 +314,10 @@ def decode_step(mixed_qkv, gate, beta, conv_weight, A_log, dt_bias, config, conv
     (unrounded pre-activation, like ``conv_decode`` in GDN mode) -> recurrent
     step; windows and states go to ``write_slots`` (in place when equal).
     Returns o [B, HV, dv]."""
+    assert write_slots.ndim == 1
+    if config.num_v_heads // config.num_k_heads <= _MAX_FUSED_GROUP:
+        return _fused(mixed_qkv, None, gate, beta, conv_weight, A_log, dt_bias, config, conv_state, recurrent_state,
+                      read_slots, write_slots, out)
     B, C = mixed_qkv.shape
     assert C == config.conv_dim
     assert read_slots.shape == write_slots.shape == (B,)
@@ -334,12 +325,9 @@ def decode_step(mixed_qkv, gate, beta, conv_weight, A_log, dt_bias, config, conv
     if out is None:
         out = torch.empty(B, config.num_v_heads, config.head_v_dim, device=mixed_qkv.device, dtype=mixed_qkv.dtype)
     assert out.shape == (B, config.num_v_heads, config.head_v_dim) and out.is_contiguous()
-    if B and config.num_v_heads // config.num_k_heads > _MAX_FUSED_GROUP:
+    if B:
         _stepwise(mixed_qkv, None, gate, beta, conv_weight, A_log, dt_bias, config, conv_state, recurrent_state,
                   read_slots, write_slots, B, 1, out)
-    elif B:
-        _fused(mixed_qkv, None, gate, beta, conv_weight, A_log, dt_bias, config, conv_state, recurrent_state,
-               read_slots, write_slots, B, 1, write_slots.stride(0), 0, out)
     return out
 
 
@@ -373,9 +361,8 @@ def verify_group(mixed_qkv, gate, beta, conv_weight, A_log, dt_bias, config, con
             verify_group(mixed_qkv, gate, beta, conv_weight, A_log, dt_bias, config, conv_state, recurrent_state,
                          rows[:, s0:s1].reshape(-1), base, write_slots[:, s0:s1], output)
     elif B:
-        _fused(mixed_qkv, row_indices, gate, beta, conv_weight, A_log, dt_bias, config, conv_state,
-               recurrent_state, baseline_slots, write_slots, B, T, write_slots.stride(0), write_slots.stride(1),
-               output)
+        _fused(mixed_qkv, row_indices, gate, beta, conv_weight, A_log, dt_bias, config, conv_state, recurrent_state,
+               baseline_slots, write_slots, output)
     return output
 
 

@@ -306,8 +306,11 @@ class GatedDeltaBackend(MixedForward):
         output = torch.empty(mixed_qkv.shape[0], config.num_v_heads, config.head_v_dim, dtype=mixed_qkv.dtype,
                              device=mixed_qkv.device)
         for seq_len, (rows, baseline, writes) in metadata.verify_groups.items():
+            # (the kernel reads int32 and int64 slots alike)
+            if writes.dtype not in (torch.int32, torch.int64):
+                writes = writes.to(torch.int64)
             verify_group(mixed_qkv, gate, beta, conv_weight, A_log, dt_bias, config, pool.conv_state,
-                         pool.recurrent_state, rows, baseline, writes.to(torch.int64), output)
+                         pool.recurrent_state, rows, baseline, writes, output)
         return output
 
 
