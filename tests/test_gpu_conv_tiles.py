@@ -44,3 +44,31 @@ def test_packed_front_end_equals_its_sequences_alone(total):
     want = ref.prepare_gdn(*ref.split_qkv(y[None], H, d, HV, d), gate[None], beta[None], A_log, dt_bias)
     for x, e in zip(got, want):
         assert_bf16_close(x, e[0], rel=1e-2, atol=1e-2)  # the bars of the front end's own tests
+
+
+# 512 channels a wave: v alone in its wave (2 key heads), v behind q and k in the same wave (1 key head)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("total", [1, 5, 67])
+def test_v_does_not_depend_on_the_wave_it_is_in(total, dtype):
+    from logssms_amd.kernel.linear_attention.fused_backend import prefill_frontend
+    from logssms_amd.layers import GatedDeltaConfig
+    g = gen(total)
+    HV, d = 2, 128
+    v_in = randn(total, HV * d, g=g, dtype=dtype, std=3.0)
+    v_in[0, 3], v_in[0, 7], v_in[-1, 11] = float("inf"), float("nan"), torch.finfo(dtype).max
+    v_weight = randn(HV * d, 1, 4, g=g, dtype=dtype, std=0.5)
+    gate, beta = (randn(total, HV, g=g, dtype=dtype) for _ in range(2))
+    A_log, dt_bias = randn(HV, g=g), randn(HV, g=g)
+    cu, base = torch.tensor([0, total]), torch.tensor([-1])
+    got = []
+    for H in (1, 2):
+        cfg = GatedDeltaConfig(H, HV, d, d, (2 * H + HV) * d, 3, 0)
+        mixed = torch.cat([randn(total, 2 * H * d, g=g, dtype=dtype), v_in], 1)
+        weight = torch.cat([randn(2 * H * d, 1, 4, g=g, dtype=dtype, std=0.5), v_weight])
+        pool = torch.zeros(1, 1, cfg.conv_dim, 3, dtype=dtype)
+        out = prefill_frontend(mixed.to(DEV), gate.to(DEV), beta.to(DEV), weight.to(DEV), A_log.to(DEV),
+                               dt_bias.to(DEV), cfg, pool.to(DEV), cu.to(DEV), base.to(DEV))
+        got.append(out[2].cpu().view(torch.int16))
+    nan = got[0].view(dtype).isnan()
+    assert torch.equal(nan, got[1].view(dtype).isnan())
+    assert torch.equal(got[0][~nan], got[1][~nan])
