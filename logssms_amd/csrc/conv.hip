@@ -226,18 +226,21 @@ __global__ __launch_bounds__(kThreads) void frontend_kernel(FrontParams fp) {
 //
 // Tokens per block.  A block walks its tile serially, about 0.6 us a token
 // when alone on its CU, so a 32-token tile took 23-29 us at any T below 4096;
-// a shorter tile re-reads the W-1 rows before it (from L2).  The largest tile
-// that still gives the chip kConvBlocks blocks (2.75 per CU) is within 8 % of
-// the fastest one measured at each T (q/k pass, 2 slabs, us at tile 32 / 16 /
-// 8 / 4 / 2): T 300: 23.8 / 13.5 / 9.0 / 6.7 / 5.8; 2048: 28.9 / 15.9 / 13.1 /
-// 13.2 / 15.9; 8192: 36.8 / 30.3 / 30.8 / 35.8 / 45.0; 16384: 63.4 / 64.4 /
-// 65.7 / 70.5 / 87.8.
+// a shorter tile re-reads the W-1 rows before it (from L2).  The tile is the
+// shortest (in whole groups of 4, the window ring's period, or 2) with which
+// all blocks run at once: kConvBlocks of them, 4 of 128 VGPRs on each CU (q/k
+// pass, 2 slabs, us at tile 32 / 16 / 8 / 4 / 2: T 300: 23.8 / 13.5 / 9.0 /
+// 6.7 / 5.8; 2048: 28.9 / 15.9 / 13.1 / 13.2 / 15.9; 8192: 36.8 / 30.3 / 30.8
+// / 35.8 / 45.0; 16384: 63.4 / 64.4 / 65.7 / 70.5 / 87.8).  Against the
+// largest power of two that gave 704 blocks, front end of 4 slabs: 2600 tokens
+// 22.3 -> 20.2, 3000 23.9 -> 20.8, 5000 35.5 -> 31.0, 6001 37.0 -> 36.3; equal
+// where both tiles are (1000, 4000, 8192, 16384).
 constexpr int kVTok = 32, kVTokMin = 2;
-constexpr int64_t kConvBlocks = 704;
+constexpr int64_t kConvBlocks = 1024;
 inline int conv_tile(int64_t tokens, int64_t slabs) {
-  int tile = kVTok;
-  while (tile > kVTokMin && (tokens + tile - 1) / tile * slabs < kConvBlocks) tile /= 2;
-  return tile;
+  const int64_t least = (tokens * slabs + kConvBlocks - 1) / kConvBlocks;
+  if (least <= kVTokMin) return kVTokMin;
+  return static_cast<int>(least >= kVTok ? kVTok : (least + 3) / 4 * 4);
 }
 
 // FRONT: fused front end (q/k normalised into q_out/k_out, v into v_out, history

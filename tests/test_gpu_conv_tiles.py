@@ -10,8 +10,8 @@ from tests.gpu_util import DEV, assert_bf16_close, gen, randn
 pytestmark = pytest.mark.gpu
 
 
-# one 2048-channel slab: tiles 2 | 4 | 8 | 16 | 32 from 1, 2813, 5625, 11249 and 22497 tokens on
-@pytest.mark.parametrize("total", [2812, 2813, 5631, 11250, 22503])
+# one 2048-channel slab: tiles 2 | 4 | 8 | 12 | ... | 28 | 32 from 1, 2049, 4097, 8193, ..., 24577 and 28673 tokens on
+@pytest.mark.parametrize("total", [2048, 2049, 2812, 2813, 4097, 5631, 8193, 11250, 22503, 28672, 28673])
 def test_packed_front_end_equals_its_sequences_alone(total):
     from logssms_amd.kernel.linear_attention.fused_backend import prefill_frontend
     from logssms_amd.layers import GatedDeltaConfig
