@@ -249,8 +249,23 @@ extern "C" int gdn_prefill_split(const void* mixed, int64_t row_stride, int io_d
                                  const void* snapshot_slots, int snapshot_slots_dtype, int64_t snapshot_count,
                                  void* out, float scale, void* workspace, int64_t workspace_bytes, void* stream) {
   using namespace gdn;
-  GDN_REQUIRE(num_seqs >= 1 && total_tokens >= 1 && H > 0 && HV > 0 && HV % H == 0 && dk > 0 && dv > 0,
+  // All that the three launches ask for, before the first of them: nothing is
+  // written unless every one of them runs (and the staging holds 16-bit q, k, v).
+  GDN_REQUIRE(num_seqs >= 1 && total_tokens >= 1 && H > 0 && HV > 0 && HV % H == 0 && dk > 0 && dv > 0 && layer >= 0 &&
+                  kernel_width >= 2 && kernel_width <= 8,
               "gdn_prefill_split: bad sizes");
+  GDN_REQUIRE(mixed && weight && cu_seqlens && conv_state && gate && beta && A_log && dt_bias && state &&
+                  baseline_slots && chunk_write_slots && out,
+              "gdn_prefill_split: null input");
+  GDN_REQUIRE(snapshot_count >= 0 && snapshot_count <= 0x7fffffff &&
+                  (snapshot_count == 0 || (snapshot_rows && snapshot_slots)),
+              "gdn_prefill_split: bad snapshot list");
+  if (!((io_dtype == GDN_BF16 || io_dtype == GDN_F16) && (dk == 32 || dk == 64 || dk == 128) &&
+        (dv == 32 || dv % 64 == 0) && (state_dtype == GDN_F32 || state_dtype == io_dtype))) {
+    set_error("gdn_prefill_split: not covered (needs 16-bit io, dk in {32, 64, 128}, dv 32 or a multiple of 64, fp32 or "
+              "io-typed state)");
+    return GDN_ERR_UNSUPPORTED;
+  }
   const SplitStaging at = split_staging(num_seqs, total_tokens, H, HV, dk, dv);
   GDN_REQUIRE(workspace && workspace_bytes >= at.bytes && aligned16(workspace),
               "gdn_prefill_split: %lld bytes of 16-byte aligned workspace needed", (long long)at.bytes);

@@ -125,3 +125,30 @@ def test_fused_prefill_reports_uncovered_shapes_without_launching():
     assert b"not covered" in lib.gdn_last_error()
     assert fused(4, 128, 96) == 2
     assert lib.gdn_conv_snapshots(d, 8192, 0, d, 1, 1, 64, 8192, 4, d, 0, 0, 0, d, 1, d, 1, d, 1, 4, None) == 1
+
+
+def test_split_prefill_refuses_before_its_first_launch():
+    """gdn_prefill_split checks what all of its launches need before the first
+    one (without a GPU a launch would come back as GDN_ERR_HIP, 3); a 32-bit
+    io type would not fit the 16-bit staging."""
+    from logssms_amd import _lib
+    if not os.path.exists(_lib.LIB_PATH):
+        pytest.skip("library not built")
+    lib = _lib.lib()
+    d = 0x10000  # 16-byte aligned dummy address, never dereferenced
+
+    def split(io=1, width=4, dk=128, dv=128, state=d, state_dtype=0, layer=0, writes=d, rows=d, slots=d, count=1,
+              out=d, base=d, workspace=d):
+        return lib.gdn_prefill_split(d, 8192, io, d, width, d, 1, 1, 1000, 16, 32, dk, dv, d, 24576, 24576, d, 32, 1,
+                                     1, d, 32, 1, 1, d, 0, d, 0, state, state_dtype, 1 << 19, 1 << 19, 1 << 14, layer,
+                                     base, 1, writes, 1, rows, 1, slots, 1, count, out, 0.1, workspace, 1 << 40, None)
+
+    for kw in (dict(io=0), dict(io=0, state_dtype=0), dict(io=7), dict(dk=256), dict(dk=48), dict(dv=96), dict(dv=16),
+               dict(state_dtype=2), dict(io=2, state_dtype=1)):
+        assert split(**kw) == 2, kw
+        assert b"gdn_prefill_split" in lib.gdn_last_error()
+    for kw in (dict(width=1), dict(width=9), dict(state=None), dict(writes=None), dict(out=None), dict(base=None),
+               dict(rows=None), dict(slots=None), dict(count=-1), dict(layer=-1), dict(workspace=None),
+               dict(workspace=d + 8)):
+        assert split(**kw) == 1, kw
+        assert b"gdn_prefill_split" in lib.gdn_last_error()
