@@ -27,6 +27,7 @@
 // Decode is HBM-bound: per (sequence, v-head) the work state (dk dv elements)
 // and n logged (k, v') rows are read; one log row, and every 16th token the
 // state, are written.
+#include <algorithm>
 #include <type_traits>
 
 #include "common.hpp"
@@ -341,17 +342,24 @@ struct ConvWindowParams {
   float s0, s1, s2;
 };
 
-// grid (tiles of kWindowTile packed rows, channel blocks).  Few rows write a
-// window (one per granule and a sequence's last), so a lane looks up one row of
-// the tile, a ballot finds the rows that write, and the block walks those with
-// its threads on the channels.  Bound: HBM latency and the bytes of the
-// windows written (one block per (row, channel block), most of which had
-// nothing to do, took 140 us for 6001 tokens x 8192 channels and 201 windows;
-// this form 9.3 us).
+// grid (tiles of kWindowTile packed rows, channel blocks, strands).  Few rows
+// write a window (one per granule and a sequence's last), so a lane looks up
+// one row of the tile, a ballot finds the rows that write, and the block walks
+// every strands-th of those with its threads on the channels.  Bound: HBM
+// latency and the bytes of the windows written (one block per (row, channel
+// block), most of which had nothing to do, took 140 us for 6001 tokens x 8192
+// channels and 201 windows; this form 9.3 us).
+// Strands: a row costs its block some 1.4 us of dependent loads, so the rows
+// of a tile are spread over as many blocks as keep the grid within
+// kWindowBlocks, all resident at once (8192 channels, us, every row writing,
+// one block / this: 32 rows 45.1 / 5.2, 300 50.5 / 10.2, 1000 56.0 / 18.9, 4096
+// 77.3 / 60.0; every 16th row: 300 rows 5.1 / 3.9, 4096 8.2 / 7.7; equal for one
+// window and from some 6000 rows on, where the tiles fill the grid).
 // VEC: 8 consecutive channels per thread, 16-byte accesses (width 4, one frame
 // per snapshot, unit input column stride, 16-byte aligned rows; checked by the
 // host): the 8 windows ([channel][tap]) are 48 contiguous bytes.
 constexpr int kWindowTile = 32;
+constexpr int64_t kWindowBlocks = 1024;
 template <class T, bool VEC>
 __global__ __launch_bounds__(kDecodeThreads) void conv_windows_frames_kernel(ConvWindowParams p) {
   const int lane = threadIdx.x & 63;
@@ -373,9 +381,10 @@ __global__ __launch_bounds__(kDecodeThreads) void conv_windows_frames_kernel(Con
   const T* x = static_cast<const T*>(p.x);
   T* st = static_cast<T*>(p.storage);
   const int64_t e0 = p.layer * p.C * p.S + ch * p.S;
-  while (rows) {
+  for (unsigned i = 0; rows; ++i) {
     const int b = __builtin_ctzll(rows);
     rows &= rows - 1;
+    if (i % gridDim.z != blockIdx.z) continue;
     const int64_t t = t0 + b;
     const int64_t n = __shfl(my_n, b), begin = __shfl(my_begin, b);
     const int64_t slot = __shfl(my_slot, b), granule = __shfl(my_gran, b), fin = __shfl(my_fin, b);
@@ -1748,8 +1757,9 @@ extern "C" int gdn_conv_windows_logstate(const void* x, int64_t x_row_stride, in
   const bool vec = kernel_width == 4 && frames_per_granule == 1 && x_col_stride == 1 && x_row_stride % 8 == 0 &&
                    channels % 8 == 0 && fe % 8 == 0 && aligned16(x) && aligned16(history) && aligned16(storage);
   const int64_t per_block = kDecodeThreads * (vec ? 8 : 1);
-  const dim3 grid(static_cast<unsigned>((total_tokens + kWindowTile - 1) / kWindowTile),
-                  static_cast<unsigned>((channels + per_block - 1) / per_block));
+  const int64_t tiles = (total_tokens + kWindowTile - 1) / kWindowTile, columns = (channels + per_block - 1) / per_block;
+  const int64_t strands = std::clamp<int64_t>(kWindowBlocks / (tiles * columns), 1, kWindowTile);
+  const dim3 grid(static_cast<unsigned>(tiles), static_cast<unsigned>(columns), static_cast<unsigned>(strands));
   auto s = static_cast<hipStream_t>(stream);
   auto launch = [&](auto type) {
     using T = decltype(type);

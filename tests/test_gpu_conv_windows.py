@@ -67,3 +67,56 @@ def test_conv_windows_match_oracle(case, scaled, dtype):
                                             frame_table=table.to(DEV), frame_bytes=frame, layer=layer),
                           width, **scale)
     assert torch.equal(dev.cpu(), want)
+
+
+def _dense(T, C, g, share=1.0):
+    """Inputs of one sequence of T rows of which a share writes a window to a slot of its own."""
+    from logssms_amd.kernel.linear_attention.packed_conv import PackedConvStateIO
+    x, hist = (randn(*s, g=g, dtype=torch.bfloat16) for s in ((T, C), (1, C, 3)))
+    slots = torch.where(torch.rand(T, generator=g) < share, torch.randperm(T, generator=g), -1).to(torch.int32)
+    storage = torch.zeros(T, C * 3, dtype=torch.bfloat16, device=DEV)
+    table = torch.arange(T, dtype=torch.int32).view(T, 1, 1)
+    io = PackedConvStateIO(storage=storage, slots=slots.to(DEV), granules=torch.zeros(T, dtype=torch.int32, device=DEV),
+                           final_slots=None, frame_table=table.to(DEV), frame_bytes=C * 6, layer=0)
+    return x, hist, slots, io
+
+
+# the rows of a tile over 32, 8 and 7 blocks and over one (8 channels per thread: 1024 / (tiles x column blocks))
+@pytest.mark.parametrize("T,C,share", [(33, 2056, 1.0), (2048, 2056, 0.5), (1153, 8200, 1.0), (16385, 2056, 0.2)])
+def test_rows_of_a_tile_spread_over_blocks(T, C, share):
+    from logssms_amd.kernel.linear_attention.packed_conv import conv_windows_logstate
+    x, hist, slots, io = _dense(T, C, gen(T), share)
+    conv_windows_logstate(x.to(DEV), hist.to(DEV), torch.tensor([0, T], device=DEV), io, 4)
+    rows = torch.cat([hist[0].t(), x])  # window of row t: the 3 rows ending at t
+    want = torch.zeros(T, C, 3, dtype=torch.bfloat16)
+    on = slots >= 0
+    want[slots[on].long()] = torch.stack([rows[1:T + 1], rows[2:T + 2], rows[3:T + 3]], 2)[on]
+    assert torch.equal(io.storage.cpu().view(T, C, 3), want)
+
+
+def test_every_row_of_a_tile_takes_little_more_than_one():
+    """32 windows in one tile: walked by one block they took 12 times as long as one (45 us against 3.6)."""
+    from logssms_amd.kernel.linear_attention.packed_conv import conv_windows_logstate
+
+    def us(only_last):
+        x, hist, slots, io = _dense(32, 8192, gen(5))
+        x, hist, cu = x.to(DEV), hist.to(DEV), torch.tensor([0, 32], device=DEV)
+        if only_last:
+            io.slots[:-1] = -1
+        conv_windows_logstate(x, hist, cu, io, 4)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            for _ in range(20):
+                conv_windows_logstate(x, hist, cu, io, 4)
+        times = []
+        for _ in range(9):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            graph.replay()
+            b.record()
+            torch.cuda.synchronize()
+            times.append(a.elapsed_time(b))
+        return sorted(times)[4] * 1e3 / 20
+
+    one, every = us(True), us(False)
+    assert every < 4 * one, f"{every:.1f} us for 32 rows, {one:.1f} us for one"
