@@ -10,6 +10,7 @@
 #include <type_traits>
 
 #include "common.hpp"
+#include "conv_tile.hpp"
 
 namespace gdn {
 namespace {
@@ -224,29 +225,16 @@ __global__ __launch_bounds__(kThreads) void frontend_kernel(FrontParams fp) {
 // and the per-head q/k sum of squares reduced across the DK/8 lanes of the
 // head with cross-lane shuffles (no LDS).
 //
-// Tokens per block.  A block walks its tile serially, about 0.6 us a token
-// when alone on its CU, so a 32-token tile took 23-29 us at any T below 4096;
-// a shorter tile re-reads the W-1 rows before it (from L2).  The tile is the
-// shortest (in whole groups of 4, the window ring's period, or 2) with which
-// all blocks run at once: kConvBlocks of them, 4 of 128 VGPRs on each CU (q/k
-// pass, 2 slabs, us at tile 32 / 16 / 8 / 4 / 2: T 300: 23.8 / 13.5 / 9.0 /
-// 6.7 / 5.8; 2048: 28.9 / 15.9 / 13.1 / 13.2 / 15.9; 8192: 36.8 / 30.3 / 30.8
-// / 35.8 / 45.0; 16384: 63.4 / 64.4 / 65.7 / 70.5 / 87.8).  Against the
-// largest power of two that gave 704 blocks, front end of 4 slabs: 2600 tokens
-// 22.3 -> 20.2, 3000 23.9 -> 20.8, 5000 35.5 -> 31.0, 6001 37.0 -> 36.3; equal
-// where both tiles are (1000, 4000, 8192, 16384).
-constexpr int kVTok = 32, kVTokMin = 2;
-constexpr int64_t kConvBlocks = 1024;
-inline int conv_tile(int64_t tokens, int64_t slabs) {
-  const int64_t least = (tokens * slabs + kConvBlocks - 1) / kConvBlocks;
-  if (least <= kVTokMin) return kVTokMin;
-  return static_cast<int>(least >= kVTok ? kVTok : (least + 3) / 4 * 4);
-}
+// Blocks of 256 threads that fit a CU, which the tile (conv_tile.hpp) counts on
+// and the launch bounds hold the registers to: 152 VGPRs for the plain bf16 conv
+// of width 4 and 129 for the front end of 256-channel heads, at most 128 elsewhere.
+template <class T, int W, int DK, bool FRONT>
+constexpr int kConvBlocks = std::is_same_v<T, bf16> && W == 4 && (!FRONT || DK == 256) ? 3 : 4;
 
 // FRONT: fused front end (q/k normalised into q_out/k_out, v into v_out, history
 // from the pool); otherwise the plain packed conv into conv.out.
 template <class T, int W, int DK, bool FRONT>
-__global__ __launch_bounds__(256) void conv_vec_kernel(FrontParams fp) {
+__global__ __launch_bounds__(256, (kConvBlocks<T, W, DK, FRONT>)) void conv_vec_kernel(FrontParams fp) {
   const ConvParams& p = fp.conv;
   constexpr int S = W - 1;
   const int64_t ch0 = (static_cast<int64_t>(blockIdx.y) * 256 + threadIdx.x) * 8;
@@ -471,10 +459,12 @@ int launch_vec(FrontParams fp, int dk, hipStream_t s) {
                        (FRONT || (reinterpret_cast<uintptr_t>(p.out) & 15) == 0) && p.W >= 2 && p.W <= 4;
   if (!aligned) return -1;
   const int64_t slabs = (p.C / 8 + 255) / 256;
-  fp.tile = conv_tile(p.T, slabs);
-  dim3 grid(static_cast<unsigned>((p.T + fp.tile - 1) / fp.tile), static_cast<unsigned>(slabs));
   auto go = [&](auto Wc, auto DKc) {
     constexpr int Wv = decltype(Wc)::value, DKv = decltype(DKc)::value;
+    // (waves past the last channel end at once: their places count for up to 4 blocks a CU)
+    const int64_t waves = (p.C / 8 + 63) / 64, fit = kConvBlocks<T, Wv, DKv, FRONT> * 4 * slabs / waves;
+    fp.tile = conv_tile(p.T, slabs, static_cast<int>(fit < 4 ? fit : 4));
+    const dim3 grid(static_cast<unsigned>((p.T + fp.tile - 1) / fp.tile), static_cast<unsigned>(slabs));
     hipLaunchKernelGGL((conv_vec_kernel<T, Wv, DKv, FRONT>), grid, dim3(256), 0, s, fp);
   };
   auto by_dk = [&](auto Wc) {
