@@ -201,11 +201,25 @@ extern "C" int gdn_chunk_gated_delta_rule_logged(
       log_dtype, token_offsets, offsets_dtype, key_heads, num_layers, page_size, out, scale, nullptr, 0, stream);
 }
 
+// A caller of the rule alone pays for a workspace and a second launch, some 4 us
+// of host time against one launch: below 6 chunks of 128-wide heads, 7 of
+// narrower ones (2.2 and 1.75 us of the one-launch chain each), that is more
+// than the GPU gains.  us a call, one launch / two, launched one after another
+// and, in brackets, replayed from a graph: 1 x 128 x 4 heads of 64 15.4 / 19.8
+// [9.0 / 9.2], 320 15.6 / 19.3 [14.4 / 11.8], 448 18.9 / 19.3 [17.8 / 13.3], 512
+// 20.1 / 19.0 [19.5 / 13.8]; 1 x 320 x 16 heads of 128 18.1 / 19.9 [17.5 / 14.3],
+// 384 19.9 / 19.5 [19.7 / 15.1].  (gdn_prefill_split makes all of its launches in
+// one call.)
+static int64_t min_rule_tokens(int64_t dk) { return dk >= 128 ? 384 : 448; }
+
 extern "C" int64_t gdn_chunk_workspace_bytes(int64_t num_seqs, int64_t total_tokens, int64_t H, int64_t HV,
                                              int64_t dk, int64_t dv, int logging) {
   if (num_seqs < 1 || total_tokens < 1 || H < 1 || HV < 1 || dk < 1 || dv < 1) return 0;
   const int64_t bytes = gdn::chunk_scan_workspace(num_seqs, total_tokens, HV, dv, logging != 0);
-  return gdn::chunk_scan_preferred(num_seqs, total_tokens, HV, dv) && bytes <= gdn::kMaxWorkspace ? bytes : 0;
+  return gdn::chunk_scan_preferred(num_seqs, total_tokens, HV, dv) && total_tokens >= min_rule_tokens(dk) * num_seqs &&
+                 bytes <= gdn::kMaxWorkspace
+             ? bytes
+             : 0;
 }
 
 // The split prefill: front end (q, k, v and gates in HBM), chunk records and

@@ -152,3 +152,22 @@ def test_split_prefill_refuses_before_its_first_launch():
                dict(workspace=d + 8)):
         assert split(**kw) == 1, kw
         assert b"gdn_prefill_split" in lib.gdn_last_error()
+
+
+def test_workspace_queries_where_two_launches_pay():
+    """The chunked rule alone asks for a workspace from 6 chunks a sequence on
+    (7 of heads narrower than 128; below, the second launch costs the host more
+    than the GPU gains); the split prefill, one call either way, from 2 on."""
+    from logssms_amd import _lib
+    if not os.path.exists(_lib.LIB_PATH):
+        pytest.skip("library not built")
+    lib = _lib.lib()
+    for n, h, hv, d in ((1, 1, 1, 64), (1, 2, 4, 64), (3, 2, 4, 32), (2, 2, 4, 128), (1, 8, 8, 128)):
+        least = 384 if d == 128 else 448
+        rule = [lib.gdn_chunk_workspace_bytes(n, n * t, h, hv, d, d, 0) for t in (128, least - 1, least, 4096)]
+        assert rule[:2] == [0, 0] and rule[2] > 0 and rule[3] > rule[2], (n, h, hv, d)
+        assert lib.gdn_prefill_workspace_bytes(n, n * 127, h, hv, d, d) == 0
+    assert lib.gdn_prefill_workspace_bytes(1, 128, 2, 4, 64, 64) > 0
+    assert lib.gdn_chunk_workspace_bytes(1, 767, 16, 32, 128, 128, 0) == 0  # 12 tokens a one-launch workgroup
+    assert lib.gdn_chunk_workspace_bytes(1, 768, 16, 32, 128, 128, 0) > 0
+    assert lib.gdn_chunk_workspace_bytes(1, 8192, 32, 64, 128, 128, 0) == 0  # one launch fills the chip
