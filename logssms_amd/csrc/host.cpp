@@ -47,6 +47,18 @@ bool convert(PyObject* o, T*& v) {  // a device address, or None
   return true;
 }
 
+// f(args...) without the interpreter lock, as ctypes calls: a launch that waits
+// for a place in a full queue does not stop the process's other Python threads.
+struct Unlocked {
+  PyThreadState* state = PyEval_SaveThread();
+  ~Unlocked() { PyEval_RestoreThread(state); }
+};
+template <class R, class... P, class... A>
+R unlocked(R (*f)(P...), A... args) {
+  const Unlocked scope;
+  return f(args...);
+}
+
 template <auto F> struct Entry;
 template <class R, class... A, R (*F)(A...)>
 struct Entry<F> {
@@ -54,7 +66,7 @@ struct Entry<F> {
   static PyObject* invoke(PyObject* const* args, std::index_sequence<I...>) {
     std::tuple<A...> v{};
     if (!(convert(args[I], std::get<I>(v)) && ...)) return nullptr;
-    return PyLong_FromLongLong(F(std::get<I>(v)...));
+    return PyLong_FromLongLong(unlocked(F, std::get<I>(v)...));
   }
   static PyObject* call(PyObject*, PyObject* const* args, Py_ssize_t n) {
     if (n != static_cast<Py_ssize_t>(sizeof...(A))) {
@@ -145,9 +157,10 @@ PyObject* conv_recurrent(PyObject*, PyObject* const* args, Py_ssize_t n) {
         PyErr_SetString(PyExc_RuntimeError, "libgdn_mi355x kernels need tensors on a ROCm device");
         throw Failed();
       }
-      const int rc = gdn_fused_conv_recurrent(
-          mixed.data_ptr(), mixed.stride(0), mixed.stride(1), dtype_code(mixed), rows ? rows->data_ptr() : nullptr,
-          rows ? index_code(*rows) : 0, weight.data_ptr(), nullptr, static_cast<int>(state_len + 1), gate.data_ptr(),
+      const int rc = unlocked(
+          &gdn_fused_conv_recurrent, mixed.data_ptr(), mixed.stride(0), mixed.stride(1), dtype_code(mixed),
+          rows ? rows->data_ptr() : nullptr, rows ? index_code(*rows) : 0, weight.data_ptr(), nullptr,
+          static_cast<int>(state_len + 1), gate.data_ptr(),
           gate.stride(0), gate.stride(1), dtype_code(gate), beta.data_ptr(), beta.stride(0), beta.stride(1),
           dtype_code(beta), A_log.data_ptr(), dtype_code(A_log), dt_bias.data_ptr(), dtype_code(dt_bias), B, T, H, HV,
           dk, dv, conv.data_ptr(), conv.stride(0), conv.stride(1), state.data_ptr(), dtype_code(state),

@@ -2,6 +2,9 @@
 checks made before any launch.  No GPU call is made."""
 
 import os
+import sys
+import threading
+import time
 
 import pytest
 import torch
@@ -63,3 +66,33 @@ def test_decode_and_verify_check_their_tensors():
         verify_group(*a[:9], None, *a[9:], torch.zeros(2 * B, HV, d))
     with pytest.raises(AssertionError):
         verify_group(*a[:9], torch.arange(B), *a[9:], torch.zeros(2 * B, HV, d))
+
+
+def test_typed_entries_run_without_the_interpreter_lock():
+    """Another Python thread gets to run beside a loop of C calls.  (With a
+    switch interval that never ends, only a call that gives the lock up lets it:
+    the loop below gives it up nowhere else.)"""
+    entry = _lib.host().gdn_rms_norm_gated
+    args = [None, 1, 0, 128, None, 1, 32, 4096, 128, 1, None, 0, 1e-6, None, None]
+    turns, started, stop = [], threading.Event(), []
+
+    def other():
+        while not stop:
+            turns.append(1)
+            started.set()
+            time.sleep(0)  # gives the lock up and waits for it
+
+    interval = sys.getswitchinterval()
+    thread = threading.Thread(target=other, daemon=True)
+    sys.setswitchinterval(1000.0)
+    try:
+        thread.start()
+        started.wait()
+        seen, until = len(turns), time.monotonic() + 10
+        while len(turns) < seen + 2 and time.monotonic() < until:
+            assert entry(*args) == 0
+        assert len(turns) >= seen + 2
+    finally:
+        stop.append(1)
+        sys.setswitchinterval(interval)
+        thread.join()
