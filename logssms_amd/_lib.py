@@ -98,11 +98,12 @@ I32_CODE, I64_CODE = 0, 1
 _DTYPE_CODES = {torch.float32: F32_CODE, torch.bfloat16: BF16_CODE, torch.float16: F16_CODE}
 
 _lib = None
+_host = None
 
 
 def lib() -> ctypes.CDLL:
-    """Load the library once; raise if it has not been built."""
-    global _lib
+    """Load the library (``LIB_PATH``) once; raise if it has not been built."""
+    global _lib, _host
     if _lib is None:
         if not os.path.exists(LIB_PATH):
             raise RuntimeError(
@@ -119,24 +120,23 @@ def lib() -> ctypes.CDLL:
         handle.gdn_abi_version.restype = ctypes.c_int
         handle.gdn_prefill_noalloc_scratch_bytes.argtypes = []
         handle.gdn_prefill_noalloc_scratch_bytes.restype = ctypes.c_int64
-        _lib = handle
+        _lib, _host = handle, None
     return _lib
-
-
-_host = None
 
 
 def host():
     """``logssms_amd._host`` (csrc/host.cpp), the host side of the per-layer
-    calls, loaded once; raise if it has not been built."""
+    calls, loaded once and bound to the instance that ``lib`` opened; raise if
+    it has not been built."""
     global _host
-    if _host is None:
-        lib()
+    if _host is None or _lib is None:
+        handle = lib()
         try:
             from . import _host as module
         except ImportError as err:
             raise RuntimeError(f"logssms_amd/_host.so cannot be loaded ({err}): build it with `make -C logssms_amd/csrc`"
                                ) from err
+        module.bind(handle._handle)
         _host = module
     return _host
 

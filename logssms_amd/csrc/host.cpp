@@ -7,6 +7,7 @@
 // A decode step of one sequence is an 8 us kernel behind what the host does
 // to launch it: 15.8 us in Python and ctypes, 5.8 us through this module.
 #include <Python.h>
+#include <dlfcn.h>
 
 #include <utility>
 
@@ -18,6 +19,51 @@
 #include "../../include/gdn_mi355x.h"
 
 namespace {
+
+// ---------------------------------------------------------------- the library
+// This module links no libgdn_mi355x.so: bind(handle) takes the functions from
+// the one instance that the package has opened (whichever file that is), so
+// that typed entries, ctypes calls and gdn_last_error share its state.
+#define GDN_TYPED(X)                      \
+  X(gdn_prefill_frontend)                 \
+  X(gdn_prefill_qk)                       \
+  X(gdn_prefill_fused)                    \
+  X(gdn_prefill_split)                    \
+  X(gdn_prefill_workspace_bytes)          \
+  X(gdn_chunk_workspace_bytes)            \
+  X(gdn_chunk_gated_delta_rule_ws)        \
+  X(gdn_chunk_gated_delta_rule_logged_ws) \
+  X(gdn_store_chunk_log)                  \
+  X(gdn_conv_snapshots)                   \
+  X(gdn_conv_windows_logstate)            \
+  X(gdn_conv_decode)                      \
+  X(gdn_conv_decode_logstate)             \
+  X(gdn_recurrent_logstate)               \
+  X(gdn_fused_recurrent)                  \
+  X(gdn_fused_conv_recurrent)             \
+  X(gdn_logstate_restore)                 \
+  X(gdn_rms_norm_gated)
+namespace lib {
+#define GDN_POINTER(name) decltype(&::name) name = nullptr;
+GDN_TYPED(GDN_POINTER)
+GDN_POINTER(gdn_last_error)
+}  // namespace lib
+
+PyObject* bind(PyObject*, PyObject* handle) {
+  void* opened = PyLong_AsVoidPtr(handle);
+  if (!opened) {
+    if (!PyErr_Occurred()) PyErr_SetString(PyExc_ValueError, "the handle of an opened library expected");
+    return nullptr;
+  }
+  auto find = [&](auto& pointer, const char* name) {
+    pointer = reinterpret_cast<std::decay_t<decltype(pointer)>>(dlsym(opened, name));
+    if (!pointer) PyErr_Format(PyExc_RuntimeError, "%s is not in the library", name);
+    return pointer != nullptr;
+  };
+#define GDN_FIND(name) && find(lib::name, #name)
+  if (!(true GDN_TYPED(GDN_FIND) GDN_FIND(gdn_last_error))) return nullptr;
+  Py_RETURN_NONE;
+}
 
 // ---------------------------------------------------------------- typed entries
 // One Python argument as its C parameter; sets a Python error and returns
@@ -59,20 +105,26 @@ R unlocked(R (*f)(P...), A... args) {
   return f(args...);
 }
 
-template <auto F> struct Entry;
-template <class R, class... A, R (*F)(A...)>
+bool bound(bool found) {
+  if (!found) PyErr_SetString(PyExc_RuntimeError, "no library bound (logssms_amd._lib.host())");
+  return found;
+}
+
+template <auto F> struct Entry;  // F: where bind() keeps the function
+template <class R, class... A, R (**F)(A...)>
 struct Entry<F> {
   template <size_t... I>
   static PyObject* invoke(PyObject* const* args, std::index_sequence<I...>) {
     std::tuple<A...> v{};
     if (!(convert(args[I], std::get<I>(v)) && ...)) return nullptr;
-    return PyLong_FromLongLong(unlocked(F, std::get<I>(v)...));
+    return PyLong_FromLongLong(unlocked(*F, std::get<I>(v)...));
   }
   static PyObject* call(PyObject*, PyObject* const* args, Py_ssize_t n) {
     if (n != static_cast<Py_ssize_t>(sizeof...(A))) {
       PyErr_Format(PyExc_TypeError, "%zu arguments expected, %zd given", sizeof...(A), n);
       return nullptr;
     }
+    if (!bound(*F != nullptr)) return nullptr;
     return invoke(args, std::index_sequence_for<A...>{});
   }
 };
@@ -157,8 +209,9 @@ PyObject* conv_recurrent(PyObject*, PyObject* const* args, Py_ssize_t n) {
         PyErr_SetString(PyExc_RuntimeError, "libgdn_mi355x kernels need tensors on a ROCm device");
         throw Failed();
       }
+      if (!bound(lib::gdn_fused_conv_recurrent != nullptr)) throw Failed();
       const int rc = unlocked(
-          &gdn_fused_conv_recurrent, mixed.data_ptr(), mixed.stride(0), mixed.stride(1), dtype_code(mixed),
+          lib::gdn_fused_conv_recurrent, mixed.data_ptr(), mixed.stride(0), mixed.stride(1), dtype_code(mixed),
           rows ? rows->data_ptr() : nullptr, rows ? index_code(*rows) : 0, weight.data_ptr(), nullptr,
           static_cast<int>(state_len + 1), gate.data_ptr(),
           gate.stride(0), gate.stride(1), dtype_code(gate), beta.data_ptr(), beta.stride(0), beta.stride(1),
@@ -170,7 +223,7 @@ PyObject* conv_recurrent(PyObject*, PyObject* const* args, Py_ssize_t n) {
           c10::hip::getCurrentHIPStream(mixed.device().index()).stream());
       if (rc != GDN_OK) {
         PyErr_Format(rc == GDN_ERR_UNSUPPORTED ? PyExc_NotImplementedError : PyExc_RuntimeError,
-                     "gdn_fused_conv_recurrent failed (%d): %s", rc, gdn_last_error());
+                     "gdn_fused_conv_recurrent failed (%d): %s", rc, lib::gdn_last_error());
         throw Failed();
       }
     }
@@ -181,27 +234,11 @@ PyObject* conv_recurrent(PyObject*, PyObject* const* args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
-#define ENTRY(name) {#name, reinterpret_cast<PyCFunction>(&Entry<&name>::call), METH_FASTCALL, nullptr}
+#define GDN_METHOD(name) {#name, reinterpret_cast<PyCFunction>(&Entry<&lib::name>::call), METH_FASTCALL, nullptr},
 PyMethodDef kMethods[] = {
+    {"bind", &bind, METH_O, nullptr},
     {"conv_recurrent", reinterpret_cast<PyCFunction>(&conv_recurrent), METH_FASTCALL, nullptr},
-    ENTRY(gdn_prefill_frontend),
-    ENTRY(gdn_prefill_qk),
-    ENTRY(gdn_prefill_fused),
-    ENTRY(gdn_prefill_split),
-    ENTRY(gdn_prefill_workspace_bytes),
-    ENTRY(gdn_chunk_workspace_bytes),
-    ENTRY(gdn_chunk_gated_delta_rule_ws),
-    ENTRY(gdn_chunk_gated_delta_rule_logged_ws),
-    ENTRY(gdn_store_chunk_log),
-    ENTRY(gdn_conv_snapshots),
-    ENTRY(gdn_conv_windows_logstate),
-    ENTRY(gdn_conv_decode),
-    ENTRY(gdn_conv_decode_logstate),
-    ENTRY(gdn_recurrent_logstate),
-    ENTRY(gdn_fused_recurrent),
-    ENTRY(gdn_fused_conv_recurrent),
-    ENTRY(gdn_logstate_restore),
-    ENTRY(gdn_rms_norm_gated),
+    GDN_TYPED(GDN_METHOD)
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_host", nullptr, -1, kMethods, nullptr, nullptr, nullptr, nullptr};
 

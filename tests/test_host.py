@@ -2,6 +2,8 @@
 checks made before any launch.  No GPU call is made."""
 
 import os
+import shutil
+import subprocess
 import sys
 import threading
 import time
@@ -96,3 +98,53 @@ def test_typed_entries_run_without_the_interpreter_lock():
         stop.append(1)
         sys.setswitchinterval(interval)
         thread.join()
+
+
+def test_one_library_instance(tmp_path):
+    """With ``LIB_PATH`` on another build of the library (as the stamp tools set
+    it), typed entries, ctypes calls and the error text all are of that one
+    instance, also after the package's own was in use."""
+    other = tmp_path / "libgdn_other.so"
+    shutil.copy(_lib.LIB_PATH, other)
+    program = f"""
+import shutil
+import subprocess
+import sys
+from logssms_amd import _lib
+if {{first}}:
+    _lib.host()
+    _lib._lib = None
+_lib.LIB_PATH = {str(other)!r}
+bad = [None, 1, 4, 0, None, 1, 32, 4096, 128, 1, None, 0, 1e-6, None, None]
+assert _lib.entry("gdn_rms_norm_gated")(*bad) == 1
+assert _lib.entry("gdn_rms_norm_gated") is not getattr(_lib.lib(), "gdn_rms_norm_gated")
+assert b"bad shape" in _lib.lib().gdn_last_error()
+libs = {{{{line.split()[-1] for line in open("/proc/self/maps") if "libgdn" in line}}}}
+assert {str(other)!r} in libs and len(libs) == 1 + {{first}}, libs
+"""
+    for first in (0, 1):
+        done = subprocess.run([sys.executable, "-c", program.format(first=first)], capture_output=True, text=True,
+                              cwd=os.path.dirname(os.path.dirname(_lib.LIB_PATH)))
+        assert done.returncode == 0, done.stderr
+
+
+def test_an_unbound_module_refuses():
+    program = """
+import torch
+from logssms_amd import _host
+try:
+    _host.gdn_rms_norm_gated(None, 1, 0, 128, None, 1, 32, 4096, 128, 1, None, 0, 1e-6, None, None)
+except RuntimeError as err:
+    assert "no library bound" in str(err)
+else:
+    raise SystemExit("called without a library")
+for bad, error in ((0, ValueError), ("x", TypeError)):
+    try:
+        _host.bind(bad)
+    except error:
+        continue
+    raise SystemExit(f"bound to {bad!r}")
+"""
+    done = subprocess.run([sys.executable, "-c", program], capture_output=True, text=True,
+                          cwd=os.path.dirname(os.path.dirname(_lib.LIB_PATH)))
+    assert done.returncode == 0, done.stderr
