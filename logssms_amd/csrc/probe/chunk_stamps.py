@@ -135,6 +135,8 @@ def run():
     buf = np.zeros(BLOCKS * WAVES * CHUNKS * SLOTS, dtype=np.uint64)
     if ctypes.CDLL(LIB).gdn_stamps_read(buf.ctypes.data_as(ctypes.c_void_p)) != 0:
         raise SystemExit("chunk_stamps: reading the stamps failed")
+    if not buf.any():
+        raise SystemExit("chunk_stamps: no stamp was written (another library ran)")
     a = buf.reshape(BLOCKS, WAVES, CHUNKS, SLOTS).astype(np.int64)
     simds = torch.zeros(BLOCKS * WAVES, dtype=torch.int32, device=dev)
     if ctypes.CDLL(LIB).gdn_stamps_simds(ctypes.c_void_p(simds.data_ptr()), BLOCKS,

@@ -120,6 +120,8 @@ def run():
     buf = np.zeros(BLOCKS * WAVES * HEADS * SLOTS, dtype=np.uint64)
     if ctypes.CDLL(LIB).gdn_lsstamps_read(buf.ctypes.data_as(ctypes.c_void_p)) != 0:
         raise SystemExit("logstate_stamps: reading the stamps failed")
+    if not buf.any():
+        raise SystemExit("logstate_stamps: no stamp was written (another library ran)")
     a = buf.reshape(BLOCKS, WAVES, HEADS, SLOTS).astype(np.int64)
     names = {0: "compute wave 0", 1: "compute wave 1", 2: "loading wave"}
     labels = {1: "state read + decayed", 2: "replay done", 3: "at MID", 4: "MID released", 5: "at END",
