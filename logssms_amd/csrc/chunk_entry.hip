@@ -69,6 +69,7 @@ int chunk_entry(const void* q, const void* k, const void* v, int io_dtype, const
   if (num_seqs == 0) return GDN_OK;
   GDN_REQUIRE(q && k && v && g && beta && cu_seqlens && state && read_slots && chunk_write_slots && out,
               "gdn_chunk_gated_delta_rule: null input");
+  GDN_REQUIRE(aligned16(workspace), "gdn_chunk_gated_delta_rule: the workspace must be 16-byte aligned");
   if (!((dk == 32 || dk == 64 || dk == 128) && (dv == 32 || (dv > 0 && dv % 64 == 0)))) {
     set_error("gdn_chunk_gated_delta_rule: unsupported head dims dk=%lld dv=%lld (dk in {32,64,128}, dv 32 or "
               "a multiple of 64)", (long long)dk, (long long)dv);

@@ -171,3 +171,22 @@ def test_workspace_queries_where_two_launches_pay():
     assert lib.gdn_chunk_workspace_bytes(1, 767, 16, 32, 128, 128, 0) == 0  # 12 tokens a one-launch workgroup
     assert lib.gdn_chunk_workspace_bytes(1, 768, 16, 32, 128, 128, 0) > 0
     assert lib.gdn_chunk_workspace_bytes(1, 8192, 32, 64, 128, 128, 0) == 0  # one launch fills the chip
+
+
+def test_chunked_rule_refuses_a_misaligned_workspace():
+    """The records are stored and read 16 bytes at a time (no launch is made:
+    without a GPU one would come back as GDN_ERR_HIP, 3)."""
+    from logssms_amd import _lib
+    if not os.path.exists(_lib.LIB_PATH):
+        pytest.skip("library not built")
+    lib = _lib.lib()
+    d = 0x10000  # 16-byte aligned dummy address, never dereferenced
+    shape = (d, d, d, 1, d, d, d, 1, 1, 4096, 2, 4, 128, 128)
+    for offset in (2, 4, 8):
+        assert lib.gdn_chunk_gated_delta_rule_ws(*shape, d, 0, 1 << 16, 1 << 16, 1 << 14, 0, d, 1, d, 1, None, 0, 64,
+                                                 None, 0, 0, 0, 0, 0, 0, d, None, 0.1, d + offset, 1 << 40, None) == 1
+        assert b"workspace" in lib.gdn_last_error()
+        assert lib.gdn_chunk_gated_delta_rule_logged_ws(*shape, d, 1, 0, d, 1, d, 1, None, 0, 64, d, 0, 8, 64, 1 << 16,
+                                                        1 << 15, 512, d, 0, d, 0, 2, 1, 256, d, 0.1, d + offset,
+                                                        1 << 40, None) == 1
+        assert b"workspace" in lib.gdn_last_error()
