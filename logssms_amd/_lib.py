@@ -160,9 +160,15 @@ def call(name: str, *args) -> None:
 
 def workspace(name: str, device, *sizes) -> tuple[torch.Tensor | None, int]:
     """The workspace the ``name`` query asks for (scratch of the current
-    stream's work), and its bytes: ``(None, 0)`` where none is used."""
+    stream's work), and its bytes: ``(None, 0)`` where none is used, and where
+    the device has no room for it (the call then runs without, as it can)."""
     n = entry(name)(*sizes)
-    return (torch.empty(n, dtype=torch.uint8, device=device), n) if n else (None, 0)
+    if not n:
+        return None, 0
+    try:
+        return torch.empty(n, dtype=torch.uint8, device=device), n
+    except torch.OutOfMemoryError:
+        return None, 0
 
 
 def dtype_code(dtype: torch.dtype) -> int:

@@ -100,6 +100,21 @@ def test_typed_entries_run_without_the_interpreter_lock():
         thread.join()
 
 
+def test_workspace_is_left_out_where_it_does_not_fit(monkeypatch):
+    """The one-launch forms need far less memory: a device with room for those
+    alone must still take the call."""
+    sizes = (1, 8192, 16, 32, 128, 128)
+    ws, n = _lib.workspace("gdn_prefill_workspace_bytes", "cpu", *sizes)
+    assert ws.numel() == n > 1 << 27
+
+    def no_room(*args, **kwargs):
+        raise torch.OutOfMemoryError("no room")
+
+    monkeypatch.setattr(torch, "empty", no_room)
+    assert _lib.workspace("gdn_prefill_workspace_bytes", "cpu", *sizes) == (None, 0)
+    assert _lib.workspace("gdn_chunk_workspace_bytes", "cpu", *sizes, 0) == (None, 0)
+
+
 def test_one_library_instance(tmp_path):
     """With ``LIB_PATH`` on another build of the library (as the stamp tools set
     it), typed entries, ctypes calls and the error text all are of that one
