@@ -247,8 +247,10 @@ __device__ __forceinline__ void sched_fence() { __builtin_amdgcn_sched_barrier(0
 //   output   o of chunk c - 1: reads Q, M, gates and the chain's operands of c - 1
 //   staging  writes K, A, V, gates of chunk c + 1, Q and M of chunk c, and
 //            issues the loads of chunk c + 1 + kDepth
-// so K rings over 3 buffers (the chain reads K^T of chunk c after B(c - 1) and
-// K of chunk c + 1 after B(c)), the gates over 4 and the rest over 2.
+// so everything has 2 buffers (the chain's last reads of K(c - 1), its K^T
+// fragments, come before B(c - 1)) but the gates: the output wave reads those of
+// chunk c - 1 while the chain reads chunk c's and chunk c + 1's are written (a
+// ring of 4).
 // EXT: checkpoints every 16 or 32 tokens, frame-table states and the token
 // log's v' rows (as chunk_chain_kernel's).
 template <int DK, class IOT, class ST, bool EXT>
@@ -258,7 +260,7 @@ __global__ __launch_bounds__(kScanThreads) void chunk_scan_kernel(ScanParams sp)
   constexpr int TILE = kC * LDK * 2;     // bytes of a K or Q tile
   constexpr int COLS = 16;
   constexpr int BUF = TILE + 6 * kFrag;  // a K tile and the A fragments, or a Q tile and the M fragments
-  __shared__ __align__(16) char sKA[3 * BUF];
+  __shared__ __align__(16) char sKA[2 * BUF];
   __shared__ __align__(16) char sQM[2 * BUF];
   __shared__ __align__(16) _Float16 sV[2 * kC * COLS];  // (a transpose read's four 32-byte rows: distinct banks)
   __shared__ __align__(16) float sG[4 * 256];  // a chunk's G, 2^G, 2^(G_last - G), beta
@@ -329,14 +331,13 @@ __global__ __launch_bounds__(kScanThreads) void chunk_scan_kernel(ScanParams sp)
     };
     __builtin_amdgcn_s_setprio(3);
     lds_barrier();  // chunk 0 staged
-    int kb = 0;     // K buffer of chunk c
     for (int c = 0; c < nchunks; ++c) {
-      const _Float16* K = reinterpret_cast<const _Float16*>(sKA + kb * BUF);
+      const _Float16* K = reinterpret_cast<const _Float16*>(sKA + (c & 1) * BUF);
       const _Float16* Vt = sV + (c & 1) * kC * COLS;
       const float* gt = sG + (c & 3) * 256;
       char* hx = sH + (c & 1) * KS * kFrag + lane * 16;
       char* vx = sX + (c & 1) * 2 * kFrag + lane * 16;
-      const char* A = sKA + kb * BUF + TILE + lane * 16;
+      const char* A = sKA + (c & 1) * BUF + TILE + lane * 16;
       // the first half of K goes out before the update, the rest after it (with K^T the whole would not fit)
       constexpr int KH = KS > 1 ? KS / 2 : KS;
       h8_t kf[KS][4];
@@ -466,7 +467,6 @@ __global__ __launch_bounds__(kScanThreads) void chunk_scan_kernel(ScanParams sp)
           return r;
         });
       }
-      kb = kb == 2 ? 0 : kb + 1;
       lds_barrier();  // B(c)
     }
     update();
@@ -594,10 +594,9 @@ __global__ __launch_bounds__(kScanThreads) void chunk_scan_kernel(ScanParams sp)
       ++next;
       if (next < nchunks) ra += rstep;
     };
-    int kb = 0;  // K buffer of the next chunk staged
     auto stage = [&](const Set& s, int c) __attribute__((always_inline)) {
       const int cq = c > 0 ? c - 1 : 0;
-      char* ka = sKA + kb * BUF;
+      char* ka = sKA + (c & 1) * BUF;
       char* qm = sQM + (cq & 1) * BUF;
       if (kq) {
         stage_rows<DK, LDK, IOT>(reinterpret_cast<_Float16*>(ka), st, s.k);
@@ -612,7 +611,6 @@ __global__ __launch_bounds__(kScanThreads) void chunk_scan_kernel(ScanParams sp)
       if (st < 64) *reinterpret_cast<uint4*>(sG + (c & 3) * 256 + 4 * st) = s.g;
       if (st == 64) sSlot[c & 3] = s.cw;
       if (EXT && st >= 128 && st < 160) *reinterpret_cast<uint4*>(sLog + (c & 1) * kC + 2 * (st & 31)) = s.log;
-      kb = kb == 2 ? 0 : kb + 1;
     };
     issue(set[0], true);
     stage(set[0], 0);
