@@ -199,7 +199,8 @@ int gdn_chunk_gated_delta_rule_logged_ws(const void* q, const void* k, const voi
                                          const void* token_offsets, int offsets_dtype, int64_t key_heads,
                                          int64_t num_layers, int64_t page_size, void* out, float scale,
                                          void* workspace, int64_t workspace_bytes, void* stream);
-/* Workspace with which the chunked rule is faster, or 0 where it is not (logging: the _logged form). */
+/* Workspace with which a call of the chunked rule is faster, the host's part included, or 0 where it is not
+ * (logging: the _logged form). */
 int64_t gdn_chunk_workspace_bytes(int64_t num_seqs, int64_t total_tokens, int64_t H, int64_t HV, int64_t dk,
                                   int64_t dv, int logging);
 
@@ -445,8 +446,8 @@ int gdn_prefill_fused(const void* q, const void* k, const void* mixed, int64_t r
  * The same prefill for few sequences, in one call: gdn_prefill_frontend, the
  * chunked rule with a workspace and gdn_conv_snapshots, with the front end's
  * outputs in the workspace too (at least gdn_prefill_workspace_bytes(...), 0
- * where gdn_prefill_qk + gdn_prefill_fused are faster).  Arguments as there;
- * same results bit for bit.
+ * where gdn_prefill_qk + gdn_prefill_fused are faster).  Arguments as there,
+ * all checked before the first launch; same results bit for bit.
  */
 int gdn_prefill_split(const void* mixed, int64_t row_stride, int io_dtype, const void* weight, int kernel_width,
                       const void* cu_seqlens, int cu_dtype, int64_t num_seqs, int64_t total_tokens, int64_t H,

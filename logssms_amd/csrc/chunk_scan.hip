@@ -23,9 +23,11 @@
 // in the workgroup, and 1.22 us with the other waves' loads and LDS traffic
 // beside it (LDS active 35 % of the cycles, no conflicts; deeper prefetch, a
 // warmed L2 and tiles laid out contiguously for the staging waves changed
-// nothing or cost their own writes).  One sequence of 8192 tokens, 16 / 32
-// heads of 128: 31 + 156 us for both launches against 286 us in one; the
-// prefill 313 -> 252 us (with v written out by the front end).  16 columns a
+// nothing or cost their own writes).  With frame tables and a token log (EXT)
+// 1.9 us a chunk: a checkpoint inside it, the v' rows' stores, and some 100 SGPR
+// spills at d_k 128 (14 without EXT).  One sequence of 8192 tokens, 16 / 32 heads
+// of 128: 165 us for both launches against 290 us in one; the prefill 312 -> 228
+// us (with v written out by the front end), replayed from a graph.  16 columns a
 // workgroup: 32 took 10 % longer for one sequence and gained only where the
 // one-launch form is the better one anyway.
 #include <type_traits>
@@ -658,12 +660,15 @@ int64_t chunk_scan_workspace(int64_t num_seqs, int64_t total_tokens, int64_t HV,
 // The scan's workgroups (16 columns each) must fit the 256 CUs at one apiece,
 // which is where the one-launch form leaves three CUs of four idle; beyond
 // that its parallel launches, whose time grows with all tokens, cost more than
-// the shorter chain saves (us, one launch / two; heads of 128, prefill: 1 x
-// 8192 x 32 heads 313 / 252, 2 x 4096 x 32 186 / 222, 2 x 8000 x 16 313 / 239,
-// 4 x 4096 x 16 220 / 247).  Below about 12 tokens a sequence and one-launch
-// workgroup the extra launches are not earned back (1 x 700 x 32 heads 43.6 /
-// 43.6, 1 x 1000 56.3 / 49.7, 1 x 300 x 16 heads 26.6 / 25.2; heads of 64: 1 x
-// 150 x 4 20.6 / 19.5, 16 x 200 x 4 32.0 / 30.5, 16 x 2500 x 4 155 / 121).
+// the shorter chain saves.  Whole prefill, replayed from a graph, us, one launch
+// / two, heads of 128: 1 x 8192 x 32 heads 312 / 228, 2 x 8000 x 16 305 / 228, but
+// 2 x 4096 x 32 184 / 233, 4 x 4096 x 16 184 / 236.  From about 12 tokens a sequence
+// and one-launch workgroup on two launches win by 10 % and more (1 x 768 x 32
+// 44.8 / 40.5, 1 x 1000 x 32 54.0 / 46.3, 2 x 800 x 16 48.5 / 42.6; heads of 64: 16
+// x 800 x 4 58.0 / 53.1, 16 x 2500 x 4 131 / 105).  Below, the two are within 7 % of
+// each other (1 x 128 x 32 19.8 / 20.3, 1 x 300 x 32 26.5 / 26.2, 1 x 500 x 32 33.6 /
+// 33.4, 1 x 700 x 32 42.4 / 39.9, 1 x 300 x 16 26.0 / 24.2, 16 x 200 x 4 of 64 26.6 /
+// 26.5), and one launch needs no workspace.
 bool chunk_scan_preferred(int64_t num_seqs, int64_t total_tokens, int64_t HV, int64_t dv) {
   const int64_t groups = num_seqs * HV * ((dv + 63) / 64);  // workgroups of the one-launch form
   const int64_t least = 12 * groups > 128 ? 12 * groups : 128;

@@ -341,7 +341,9 @@ __global__ __launch_bounds__(256, (kConvBlocks<T, W, DK, FRONT>)) void conv_vec_
   // Whether the wave holds v channels alone (lane 0 has its smallest): its
   // values are packed as they come, without the q/k head sums and the rounding
   // to floats between, 26 of some 115 VALU instructions a token (16 / 32 heads
-  // of 128: 8192 tokens 60 -> 56 us, 6001 tokens 50.4 -> 49.3).
+  // of 128, kernel traces of whole prefills, whose inputs come from HBM: one
+  // prompt of 8192 tokens 60 -> 56 us; 6001 tokens of a LogState prefill, at 32
+  // tokens a tile, 50.4 -> 49.3, and 44.3 at the 24 it takes now).
   const bool v_wave = FRONT && __builtin_amdgcn_readfirstlane(static_cast<int>(ch0)) >= 2 * key_dim;
   // The outputs of token t (ALL: every lane of the block is active).
   auto emit = [&](int64_t t, float (&y)[8], auto all) __attribute__((always_inline)) {
